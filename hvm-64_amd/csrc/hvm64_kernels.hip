@@ -207,7 +207,35 @@ DEV void wave_sleep(u32 units) {
   for (u32 z = 0; z < units; z++) __builtin_amdgcn_s_sleep(2);
 }
 
+// Wave-wide values for the scheduler.  A loop pass reads about twenty of
+// them; through LDS (ds_bpermute, what __shfl compiles to) each costs its
+// round trip of 100+ cycles, and a wave that is alone on its SIMD has nothing
+// to run meanwhile.  Lane 0's value and a lane at a wave-uniform index are
+// register reads; sums and maxima over the lanes of row 0 (the ring classes,
+// NCLS <= 16) are four DPP row shifts.  Measured through LDS and then this
+// way: Church c2^c9, one busy wave, 5.38 -> 5.05 ms; bitonic 2^6 8.31 -> 8.19.
 DEV u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+DEV u64 uniform(u64 v) { return (u64)uniform((u32)v) | (u64)uniform((u32)(v >> 32)) << 32; }
+DEV u32 lane_at(u32 v, u32 i) { return __builtin_amdgcn_readlane(v, i); }
+DEV u64 lane_at(u64 v, u32 i) { return (u64)lane_at((u32)v, i) | (u64)lane_at((u32)(v >> 32), i) << 32; }
+// The value n lanes below in the row of 16 (0 beyond its edge).
+template <u32 n>
+DEV u32 row_below(u32 v) { return __builtin_amdgcn_update_dpp(0, v, 0x110 + n, 0xF, 0xF, true); }
+DEV u32 row0_sum(u32 v) {
+  v += row_below<1>(v);
+  v += row_below<2>(v);
+  v += row_below<4>(v);
+  v += row_below<8>(v);
+  return lane_at(v, 15);
+}
+DEV u32 row0_max(u32 v) {
+  u32 o;
+  o = row_below<1>(v), v = o > v ? o : v;
+  o = row_below<2>(v), v = o > v ? o : v;
+  o = row_below<4>(v), v = o > v ? o : v;
+  o = row_below<8>(v), v = o > v ? o : v;
+  return lane_at(v, 15);
+}
 
 // Moves `cnt` redexes, the oldest of class `c`, from the wave's rings to the
 // global ring (all lanes; lane 0 updates the counters).  Returns S after.
@@ -216,7 +244,7 @@ DEV u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
 DEV void claim_global(const Params &P, Lane &L, u64 *bag, u32 *top_c, u32 k, u32 lane, u64 t_end) {
   u64 base = 0;
   if (lane == 0) base = __hip_atomic_fetch_add(&P.g->q_head, (u64)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  base = __shfl(base, 0, 64);
+  base = uniform(base);
   if (lane < k) {
     u64 *slot = P.queue + ((base + lane) & P.qmask) * 2;
     u64 a, b;
@@ -247,7 +275,7 @@ DEV u64 spill_to_global(const Params &P, u64 *bag, u32 *bot_c, u32 c, u32 cnt, u
   publish();
   u64 base = 0;
   if (lane == 0) base = __hip_atomic_fetch_add(&P.g->q_tail, (u64)cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  base = __shfl(base, 0, 64);
+  base = uniform(base);
   for (u32 i = lane; i < cnt; i += 64) {
     u32 s2 = (ring_base(c) + ((bot + i) & (ring_cap(c) - 1))) * 2;
     u64 *q = P.queue + ((base + i) & P.qmask) * 2;
@@ -261,7 +289,7 @@ DEV u64 spill_to_global(const Params &P, u64 *bag, u32 *bot_c, u32 c, u32 cnt, u
     if ((old >> 32) + cnt > (P.qmask + 1) / 2) err = ERR_QUEUE;
     *bot_c = bot + cnt;
   }
-  return __shfl(old, 0, 64) + ((u64)cnt << 32);
+  return uniform(old) + ((u64)cnt << 32);
 }
 
 // Serving: wave 0 admits waiting requests, one per lane (at most 64, and at
@@ -285,10 +313,10 @@ DEV u32 serve_admit(const Params &P, Lane &L, u32 lane, u64 t_end) {
       HVM_ST(&sv[SV_REQ_HEAD], head + k);
     }
   }
-  k = __shfl(k, 0, 64);
+  k = uniform(k);
   if (k == 0) return 0;
-  head = __shfl(head, 0, 64);
-  fhead = __shfl(fhead, 0, 64);
+  head = uniform(head);
+  fhead = uniform(fhead);
   if (lane < k) {
     // the entry a completing lane wrote before it counted the slot free
     u64 *slot = &P.free_ring[(fhead + lane) % P.serve_slots];
@@ -321,7 +349,7 @@ DEV bool serve_waiting(const Params &P, u32 lane) {
     const u64 tail = HVM_LD_SYS(&P.host_ctl[SH_REQ_TAIL]);
     w = tail > HVM_LD(&P.serve_ctl[SV_REQ_HEAD]) && HVM_LD(&P.serve_ctl[SV_FREE_COUNT]) > 0;
   }
-  return __shfl(w, 0, 64) != 0;
+  return uniform(w) != 0;
 }
 
 // After pushes outside an iteration (admission), trim each ring whose push
@@ -420,8 +448,8 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
 
   for (;;) {
     if (fresh) {
-      S_cache = __shfl(S_next, 0, 64);
-      u32 err = __shfl(err_next, 0, 64);
+      S_cache = uniform(S_next);
+      u32 err = uniform(err_next);
       fresh = false;
       if (err) {
         if (SERVE && lane == 0) HVM_ST_SYS(&P.host_ctl[SH_ERR], (u64)err);
@@ -444,10 +472,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // ring occupancy: lane c < NCLS reads class c
     u32 my_top = lane < NCLS ? top_c[lane] : 0, my_bot = lane < NCLS ? bot_c[lane] : 0;
     u32 my_n = my_top - my_bot;
-    u32 n = my_n;
-#pragma unroll
-    for (u32 o = 1; o < 16; o <<= 1) n += __shfl_xor(n, o, 64);
-    n = uniform(n);
+    u32 n = row0_sum(my_n);
 
     // ---- empty rings: idle.  An idle wave is in the idle set (its bit in
     // P.idle_bits) and polls its own mailbox, where a busy wave can hand it
@@ -462,7 +487,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
         in_set = use_mbox;
         u64 old = 0;
         if (lane == 0) old = __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        S_cache = __shfl(old, 0, 64) - 1;
+        S_cache = uniform(old) - 1;
         active = false;
         idle_polls = 0;
         // nothing active, nothing queued: done (serving: once the host has
@@ -471,7 +496,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
         if (SERVE && end) {
           u64 stop = 0;
           if (lane == 0) stop = HVM_LD_SYS(&P.host_ctl[SH_STOP]);
-          end = __shfl(stop, 0, 64) != 0;
+          end = uniform(stop) != 0;
         }
         if (end) {
           // no wave is active, so no delivery is in flight: tell the idle
@@ -485,7 +510,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
       if (use_mbox) {
         u64 k = 0;
         if (lane == 0) k = gld(my_box);
-        k = __shfl(k, 0, 64);
+        k = uniform(k);
         if (k == MBOX_DONE) break;
         if (k > 0) {  // a delivery: the sender already counted this wave active
           if (lane < k) {
@@ -517,7 +542,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           if (lane == 0)
             old = __hip_atomic_fetch_and(&P.idle_bits[gwave >> 6], ~(1ull << (gwave & 63)), __ATOMIC_RELAXED,
                                          __HIP_MEMORY_SCOPE_AGENT);
-          left = ((__shfl(old, 0, 64) >> (gwave & 63)) & 1) != 0;
+          left = ((uniform(old) >> (gwave & 63)) & 1) != 0;
           in_set = false;  // either we left, or a sender took us out and a delivery is coming
         }
         if (left) {
@@ -537,9 +562,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           err = gld32(&g->err);
           if (SERVE) stop = (u32)HVM_LD_SYS(&P.host_ctl[SH_STOP]);
         }
-        s = __shfl(s, 0, 64);
-        err = __shfl(err, 0, 64);
-        stop = __shfl(stop, 0, 64);
+        s = uniform(s);
+        err = uniform(err);
+        stop = uniform(stop);
         S_cache = s;
         if (err) {
           if (SERVE && lane == 0) HVM_ST_SYS(&P.host_ctl[SH_ERR], (u64)err);
@@ -559,7 +584,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
             if (lane == 0)
               old = __hip_atomic_fetch_and(&P.idle_bits[gwave >> 6], ~(1ull << (gwave & 63)), __ATOMIC_RELAXED,
                                            __HIP_MEMORY_SCOPE_AGENT);
-            left = ((__shfl(old, 0, 64) >> (gwave & 63)) & 1) != 0;
+            left = ((uniform(old) >> (gwave & 63)) & 1) != 0;
             in_set = false;  // either we left, or a sender took us out and a delivery is coming
           }
           if (left) {
@@ -577,7 +602,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
                 }
               }
             }
-            k = __shfl(k, 0, 64);
+            k = uniform(k);
             if (k > 0) {
               backoff = 1 + (gwave & 7);
               active = true;
@@ -610,16 +635,11 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // definition calls meanwhile gather into fuller iterations), else the
     // fullest definition-call ring; lowest index on ties
     u32 key = lane < NCLS ? ((lane < CLS_CALL && my_n > 0) ? (1u << 24) : 0u) | (my_n << 4) | (15 - lane) : 0;
-#pragma unroll
-    for (u32 o = 1; o < 16; o <<= 1) {
-      u32 other = __shfl_xor(key, o, 64);
-      key = other > key ? other : key;
-    }
-    key = uniform(key);
+    key = row0_max(key);
     const u32 c = 15 - (key & 15);
     const u32 nc = (key >> 4) & 0xFFFFF;
-    const u32 top = uniform(__shfl(my_top, c, 64));
-    const u32 bot = uniform(__shfl(my_bot, c, 64));
+    const u32 top = lane_at(my_top, c);
+    const u32 bot = lane_at(my_bot, c);
 
     // ---- budget for reduce(limit) (net.rs:41-52)
     u32 take = nc < 64 ? nc : 64;
@@ -640,12 +660,12 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           }
         }
       }
-      take = uniform(__shfl(granted, 0, 64));
+      take = uniform(granted);
       if (take == 0) {
         // budget spent: hand every ring back to the global queue and stop
         u32 qerr = 0;
         for (u32 cc = 0; cc < NCLS; cc++) {
-          u32 t2 = uniform(__shfl(my_top, cc, 64)), b2 = uniform(__shfl(my_bot, cc, 64));
+          u32 t2 = lane_at(my_top, cc), b2 = lane_at(my_bot, cc);
           if (t2 != b2) S_cache = spill_to_global(P, bag, &bot_c[cc], cc, t2 - b2, lane, b2, qerr);
         }
         if (qerr) fail(L, qerr);
@@ -707,17 +727,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
       top_c[lane] = my_top;
     }
     my_n = my_top - my_bot;
-    n = my_n;
-#pragma unroll
-    for (u32 o = 1; o < 16; o <<= 1) n += __shfl_xor(n, o, 64);
-    n = uniform(n);
+    n = row0_sum(my_n);
     key = lane < NCLS ? (my_n << 4) | (15 - lane) : 0;
-#pragma unroll
-    for (u32 o = 1; o < 16; o <<= 1) {
-      u32 other = __shfl_xor(key, o, 64);
-      key = other > key ? other : key;
-    }
-    key = uniform(key);
+    key = row0_max(key);
     const u32 sc = 15 - (key & 15);
     const u32 snc = key >> 4;
     u32 active_waves = (u32)(S_cache & 0xFFFFFFFFu);
@@ -742,21 +754,21 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
       const u64 ball = __ballot(w != 0);
       if (ball) {
         const u32 first = (u32)__builtin_ctzll(ball);
-        const u32 word = uniform(__shfl(wi, first, 64));
-        const u64 bits = __shfl(w, first, 64);
+        const u32 word = lane_at(wi, first);
+        const u64 bits = lane_at(w, first);
         const u32 r = gwave & 63;
         const u64 rot = (bits >> r) | (r ? bits << (64 - r) : 0);
         const u32 bit = ((u32)__builtin_ctzll(rot) + r) & 63;
         u64 old = 0;
         if (lane == 0)
           old = __hip_atomic_fetch_and(&P.idle_bits[word], ~(1ull << bit), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool got = ((__shfl(old, 0, 64) >> bit) & 1) != 0;
+        const bool got = ((uniform(old) >> bit) & 1) != 0;
         const u32 target = word * 64 + bit;
         if (got && target < P.total_waves) {
           if (lane == 0) __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           publish();  // the nodes these redexes reach, before the mailbox entries
           u64 *box = P.mbox + (u64)target * MBOX_WORDS;
-          const u32 bot0 = uniform(__shfl(my_bot, sc, 64));
+          const u32 bot0 = lane_at(my_bot, sc);
           if (lane < give) {
             const u32 s2 = (ring_base(sc) + ((bot0 + lane) & (ring_cap(sc) - 1))) * 2;
             gst(box + 16 + 2 * lane, bag[s2]);
@@ -778,7 +790,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
       if (TIMING) st[ST_SPILLS]++;
       if (TIMING) st[ST_SPILLED] += spill;
       u32 qerr = 0;
-      S_cache = spill_to_global(P, bag, &bot_c[sc], sc, spill, lane, uniform(__shfl(my_bot, sc, 64)), qerr);
+      S_cache = spill_to_global(P, bag, &bot_c[sc], sc, spill, lane, lane_at(my_bot, sc), qerr);
       if (qerr) fail(L, qerr);
       if (timing) st[ST_SPILL_TICKS] += wall_clock64() - t_sp;
     }
@@ -806,8 +818,8 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           s_new = s;
         }
       }
-      k = uniform(__shfl(k, 0, 64));
-      S_cache = __shfl(s_new, 0, 64);
+      k = uniform(k);
+      S_cache = uniform(s_new);
       if (k > 0) {
         if (TIMING) st[ST_CLAIMS]++;
         if (TIMING) st[ST_CLAIMED] += k;

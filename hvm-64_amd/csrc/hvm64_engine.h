@@ -93,7 +93,7 @@ enum : u32 { BAD_HEAP_ADDR = 1, BAD_LINK_LIST, BAD_CHAIN, BAD_RESOLVE, BAD_SLOTS
 // (keeping them costs it 2-4%); batched and serving launches always do.
 enum : u32 {
   ST_BUSY_IT = 0, ST_IDLE_IT, ST_BUSY_TICKS, ST_SPILLS, ST_SPILLED, ST_CLAIMS, ST_CLAIMED,
-  ST_INTERACT_TICKS,  // ticks inside interact() (the divergent section)
+  ST_INTERACT_TICKS,  // ticks inside the tasks (the divergent section)
   ST_SPILL_TICKS,     // ticks spilling to the global ring
   ST_CLS_IT,          // 4 slots: iterations that ran each redex class
   ST_CLS_TICKS = ST_CLS_IT + 4,  // 4 slots: ticks inside the rules, per class

@@ -52,14 +52,14 @@ __global__ void k_fill(u64 *words, u64 n, u64 value) {
 // (encode.rs:31-35, counts nothing).  Redexes go to the global ring.
 __global__ void k_exec(Params P, u32 def, u64 t0, u32 count_dref) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  __shared__ u64 s_pl[2 * LINK_CAP * 64];
+  __shared__ pair s_pl[LINK_CAP * 64];
   __shared__ u64 s_t[LDS_SLOTS * 64];
   Lane L;
   lane_init(L, P, 0, 0);
   L.PL = s_pl;
   L.T_lds = s_t;
   if (count_dref) L.rw[RW_DREF]++;
-  run_task(L, false, 0, 0, def, t0);
+  run_def(L, def, t0);
   publish();
   lane_finish(L);
   for (u32 k = 0; k < RW_SLOTS; k++)
@@ -71,7 +71,7 @@ __global__ void k_exec(Params P, u32 def, u64 t0, u32 count_dref) {
 // DREF each).  One wave per block; each lane boots nets lane, lane + 64*B,
 // ...  Redexes go to the global ring.
 __global__ __launch_bounds__(64) void k_boot_batch(Params P, u32 n, const u32 *defs, u64 *roots) {
-  __shared__ u64 s_pl[2 * LINK_CAP * 64];
+  __shared__ pair s_pl[LINK_CAP * 64];
   __shared__ u64 s_t[LDS_SLOTS * 64];
   const u32 lane = threadIdx.x;
   Lane L;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(64) void k_boot_batch(Params P, u32 n, const u32 *d
     u64 r = alloc_var1(L);
     roots[i] = r;
     L.rw[RW_DREF]++;
-    run_task(L, false, 0, 0, di, var_port(r));
+    run_def(L, di, var_port(r));
   }
   publish();
   lane_finish(L);
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64) void k_boot_batch(Params P, u32 n, const u32 *d
 
 // Net::expand for every net of a batch: roots[i] is replaced by the new root.
 __global__ __launch_bounds__(64) void k_expand_batch(Params P, u32 n, u64 *roots) {
-  __shared__ u64 s_pl[2 * LINK_CAP * 64];
+  __shared__ pair s_pl[LINK_CAP * 64];
   const u32 lane = threadIdx.x;
   Lane L;
   lane_init(L, P, blockIdx.x, lane);
@@ -107,8 +107,7 @@ __global__ __launch_bounds__(64) void k_expand_batch(Params P, u32 n, u64 *roots
     u64 old = roots[i];
     L.cur_net = i;
     u64 r2 = alloc_node(L), e = r2 + 8;
-    st2(P, r2, P_NONE, var_port(r2));
-    L.dirty = true;
+    st2(L, r2, P_NONE, var_port(r2));
     u32 np = 0;
     push_link(L, np, var_port(old), expand_ref(e));
     flush_links(L, np);
@@ -158,13 +157,12 @@ __global__ void k_root_ports(Params P, u32 n, const u64 *roots, u64 *out) {
 // to g->result.
 __global__ void k_expand(Params P, u64 old_root_cell) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  __shared__ u64 s_pl[2 * LINK_CAP * 64];
+  __shared__ pair s_pl[LINK_CAP * 64];
   Lane L;
   lane_init(L, P, 0, 0);
   L.PL = s_pl;
   u64 r2 = alloc_node(L), e = r2 + 8;
-  st2(P, r2, P_NONE, var_port(r2));
-  L.dirty = true;
+  st2(L, r2, P_NONE, var_port(r2));
   u32 np = 0;
   push_link(L, np, var_port(old_root_cell), expand_ref(e));
   flush_links(L, np);
@@ -241,7 +239,7 @@ DEV u32 row0_max(u32 v) {
 // global ring (all lanes; lane 0 updates the counters).  Returns S after.
 // Takes the next k (<= 64) redexes of the global ring, whose count in S this
 // wave has already claimed, into its rings (the caller checks they fit).
-DEV void claim_global(const Params &P, Lane &L, u64 *bag, u32 *top_c, u32 k, u32 lane, u64 t_end) {
+DEV void claim_global(const Params &P, Lane &L, pair *bag, u32 *top_c, u32 k, u32 lane, u64 t_end) {
   u64 base = 0;
   if (lane == 0) base = __hip_atomic_fetch_add(&P.g->q_head, (u64)k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   base = uniform(base);
@@ -263,13 +261,11 @@ DEV void claim_global(const Params &P, Lane &L, u64 *bag, u32 *top_c, u32 k, u32
     gst(slot + 1, 0);
     const u32 c = redex_class(a, b, L.book, has_book(L), P.ndefs);
     const u32 idx = HVM_LDS_FAA(&top_c[c], 1u);
-    const u32 i = (ring_base(c) + (idx & (ring_cap(c) - 1))) * 2;
-    bag[i] = a;
-    bag[i + 1] = b;
+    bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
   }
 }
 
-DEV u64 spill_to_global(const Params &P, u64 *bag, u32 *bot_c, u32 c, u32 cnt, u32 lane, u32 bot, u32 &err) {
+DEV u64 spill_to_global(const Params &P, const pair *bag, u32 *bot_c, u32 c, u32 cnt, u32 lane, u32 bot, u32 &err) {
   // the nodes these redexes reach must be in memory before a claimer can
   // read the ring slots (which it may do before S counts them)
   publish();
@@ -277,10 +273,10 @@ DEV u64 spill_to_global(const Params &P, u64 *bag, u32 *bot_c, u32 c, u32 cnt, u
   if (lane == 0) base = __hip_atomic_fetch_add(&P.g->q_tail, (u64)cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   base = uniform(base);
   for (u32 i = lane; i < cnt; i += 64) {
-    u32 s2 = (ring_base(c) + ((bot + i) & (ring_cap(c) - 1))) * 2;
+    const pair r = bag[ring_base(c) + ((bot + i) & (ring_cap(c) - 1))];
     u64 *q = P.queue + ((base + i) & P.qmask) * 2;
-    gst(q, bag[s2]);
-    gst(q + 1, bag[s2 + 1]);
+    gst(q, r.a);
+    gst(q + 1, r.b);
   }
   publish();
   u64 old = 0;
@@ -293,9 +289,9 @@ DEV u64 spill_to_global(const Params &P, u64 *bag, u32 *bot_c, u32 c, u32 cnt, u
 }
 
 // Serving: wave 0 admits waiting requests, one per lane (at most 64, and at
-// most as many as there are free slots), booting each into a free slot.
-// Returns how many it booted.
-DEV u32 serve_admit(const Params &P, Lane &L, u32 lane, u64 t_end) {
+// most as many as there are free slots).  True on the lanes that got one,
+// set up to boot it (serve_boot): definition di with t0.
+DEV bool serve_admit(const Params &P, Lane &L, u32 lane, u64 t_end, u32 &di, u64 &t0, u32 &np) {
   u64 *const sv = P.serve_ctl;
   u64 *const hc = P.host_ctl;
   u64 k = 0, head = 0, fhead = 0;
@@ -314,9 +310,10 @@ DEV u32 serve_admit(const Params &P, Lane &L, u32 lane, u64 t_end) {
     }
   }
   k = uniform(k);
-  if (k == 0) return 0;
+  if (k == 0) return false;
   head = uniform(head);
   fhead = uniform(fhead);
+  bool boot = false;
   if (lane < k) {
     // the entry a completing lane wrote before it counted the slot free
     u64 *slot = &P.free_ring[(fhead + lane) % P.serve_slots];
@@ -334,12 +331,18 @@ DEV u32 serve_admit(const Params &P, Lane &L, u32 lane, u64 t_end) {
       HVM_ST(slot, 0);
       const u64 *rq = P.req + ((head + lane) & P.req_mask) * 2;
       const u64 d = HVM_LD_SYS(rq), tag = HVM_LD_SYS(rq + 1);
-      if (d == 0 || d - 1 >= P.ndefs) fail(L, ERR_BADPTR, BAD_DEF_CALL);
-      else serve_boot(L, (u32)(v - 1), (u32)(d - 1), tag);
+      if (d == 0 || d - 1 >= P.ndefs) {
+        fail(L, ERR_BADPTR, BAD_DEF_CALL);
+      } else {
+        boot = true;
+        di = (u32)(d - 1);
+        t0 = serve_boot(L, (u32)(v - 1), tag, np);
+      }
     }
   }
-  if (lane == 0) HVM_ST_SYS(&hc[SH_REQ_HEAD], head + k);  // the host sees the ring's room
-  return (u32)k;
+  // the host sees the ring's room: the entries have been read
+  if (lane == 0) HVM_ST_SYS(&hc[SH_REQ_HEAD], head + k);
+  return boot;
 }
 
 // Serving: requests waiting and slots free (wave 0, lane 0's view).
@@ -350,13 +353,6 @@ DEV bool serve_waiting(const Params &P, u32 lane) {
     w = tail > HVM_LD(&P.serve_ctl[SV_REQ_HEAD]) && HVM_LD(&P.serve_ctl[SV_FREE_COUNT]) > 0;
   }
   return uniform(w) != 0;
-}
-
-// After pushes outside an iteration (admission), trim each ring whose push
-// counter ran past its capacity: those pushes went to the global ring.
-DEV void clamp_rings(u32 *top_c, const u32 *bot_c, u32 lane) {
-  if (lane < NCLS && top_c[lane] - bot_c[lane] > ring_cap(lane)) top_c[lane] = bot_c[lane] + ring_cap(lane);
-  __builtin_amdgcn_wave_barrier();
 }
 
 // ARENAS: compiled for per-net arenas (P.gmap set) or for the per-lane
@@ -370,8 +366,10 @@ DEV void clamp_rings(u32 *top_c, const u32 *bot_c, u32 lane) {
 // and P.t_lds are set), so the instantiation reads them only from there.
 template <bool ARENAS, bool SERVE, bool TIMING, bool LDS>
 __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
-  __shared__ u64 s_bag[WAVES_PER_BLOCK][RING_PAIRS * 2];
-  __shared__ u64 s_T[WAVES_PER_BLOCK][(LDS_SLOTS + 2 * LINK_CAP) * 64];
+  __shared__ pair s_bag[WAVES_PER_BLOCK][RING_PAIRS];
+  __shared__ pair s_links[WAVES_PER_BLOCK][LINK_CAP * 64];
+  __shared__ u64 s_T[WAVES_PER_BLOCK][LDS_SLOTS * 64];
+  __shared__ u64 s_cache[ARENAS ? 1 : WAVES_PER_BLOCK][ARENAS ? 1 : FREE_CACHE * 64];  // arenas reuse no node
   __shared__ u32 s_top[WAVES_PER_BLOCK][NCLS];
   __shared__ u32 s_bot[WAVES_PER_BLOCK][NCLS];
   __shared__ u64 s_book[BOOK_LDS_WORDS];
@@ -390,7 +388,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   __syncthreads();
   const u32 gwave = blockIdx.x * WAVES_PER_BLOCK + wib;
   Globals *g = P.g;
-  u64 *bag = s_bag[wib];
+  pair *bag = s_bag[wib];
   u32 *top_c = s_top[wib];
   u32 *bot_c = s_bot[wib];
   if (lane < NCLS) {
@@ -404,7 +402,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   L.serve = SERVE;
   L.lds_all = LDS;
   L.T_lds = &s_T[wib][lane];
-  L.PL = &s_T[wib][LDS_SLOTS * 64 + lane];
+  L.PL = &s_links[wib][lane];
+  L.in_lds = true;
+  L.FC = &s_cache[ARENAS ? 0 : wib][ARENAS ? 0 : lane];
   if (LDS || P.book_lds) {
     L.book = HVM_TO_LDS(s_book);
     L.book_ins = nd;
@@ -462,13 +462,14 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     }
     // ---- serving: the last task's count change (a net it completed), then
     // wave 0 admits requests every fourth busy iteration
+    // (an admitting pass boots requests instead of popping redexes)
     if (SERVE) serve_settle(L);
-    if (SERVE && gwave == 0 && active && (++admit_tick & 3) == 0) {
-      __builtin_amdgcn_wave_barrier();
-      serve_admit(P, L, lane, t_end);
-      __builtin_amdgcn_wave_barrier();
-      clamp_rings(top_c, bot_c, lane);
-    }
+    bool boot = false;
+    u32 boot_def = 0, np0 = 0;
+    u64 boot_t0 = 0;
+    if (SERVE && gwave == 0 && active && (admit_tick++ & 3) == 0)
+      boot = serve_admit(P, L, lane, t_end, boot_def, boot_t0, np0);
+    const bool admitting = SERVE && HVM_ANY(boot);
     // ring occupancy: lane c < NCLS reads class c
     u32 my_top = lane < NCLS ? top_c[lane] : 0, my_bot = lane < NCLS ? bot_c[lane] : 0;
     u32 my_n = my_top - my_bot;
@@ -479,7 +480,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // redexes directly and where the end of the reduction is announced
     // (MBOX_DONE); every IDLE_CHECK polls it also reads S, for redexes on
     // the global ring, errors and the deadline.
-    if (n == 0) {
+    if (n == 0 && !admitting) {
       if (active) {
         if (use_mbox && lane == 0)
           __hip_atomic_fetch_or(&P.idle_bits[gwave >> 6], 1ull << (gwave & 63), __ATOMIC_RELAXED,
@@ -517,9 +518,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
             const u64 a = gld(my_box + 16 + 2 * lane), b = gld(my_box + 16 + 2 * lane + 1);
             const u32 c = redex_class(a, b, L.book, has_book(L), P.ndefs);  // the rings are empty: k <= 64 entries fit
             const u32 idx = HVM_LDS_FAA(&top_c[c], 1u);
-            const u32 i = (ring_base(c) + (idx & (ring_cap(c) - 1))) * 2;
-            bag[i] = a;
-            bag[i + 1] = b;
+            bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
           }
           if (lane == 0) gst(my_box, 0);
           if (TIMING) st[ST_CLAIMS]++;
@@ -548,9 +547,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
         if (left) {
           if (lane == 0) __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           active = true;
-          serve_admit(P, L, lane, t_end);
-          __builtin_amdgcn_wave_barrier();
-          clamp_rings(top_c, bot_c, lane);
+          admit_tick = 0;  // the next pass admits
           continue;
         }
       }
@@ -636,14 +633,14 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // fullest definition-call ring; lowest index on ties
     u32 key = lane < NCLS ? ((lane < CLS_CALL && my_n > 0) ? (1u << 24) : 0u) | (my_n << 4) | (15 - lane) : 0;
     key = row0_max(key);
-    const u32 c = 15 - (key & 15);
+    const u32 c = admitting ? (u32)CLS_CALL : 15 - (key & 15);
     const u32 nc = (key >> 4) & 0xFFFFF;
     const u32 top = lane_at(my_top, c);
     const u32 bot = lane_at(my_bot, c);
 
     // ---- budget for reduce(limit) (net.rs:41-52)
-    u32 take = nc < 64 ? nc : 64;
-    if (limited) {
+    u32 take = admitting ? 0 : nc < 64 ? nc : 64;
+    if (!SERVE && limited) {
       u32 granted = 0;
       if (lane == 0) {
         u64 d = gld(&g->done);
@@ -683,17 +680,18 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     bool has = nth < take;
     u64 ra = 0, rb = 0;
     if (has) {
-      u32 i = (ring_base(c) + ((top - 1 - nth) & (ring_cap(c) - 1))) * 2;
-      ra = bag[i];
-      rb = bag[i + 1];
+      const pair r = bag[ring_base(c) + ((top - 1 - nth) & (ring_cap(c) - 1))];
+      ra = r.a;
+      rb = r.b;
     }
     rot = (rot + take) & 63;
     __builtin_amdgcn_wave_barrier();
     if (lane == 0) top_c[c] = top - take;
     __builtin_amdgcn_wave_barrier();
     const u64 t_in = timing ? wall_clock64() : 0;
-    if (has) L.rw[RW_POPS]++;
-    run_task(L, has, ra, rb, NO_DEF, 0);
+    L.rw[RW_POPS] += has;
+    run_tasks(L, c, has, ra, rb, boot, boot_def, boot_t0, np0);
+    if (SERVE && (has || boot)) serve_account_deferred(L, L.pushed - 1u);
     {
       const u64 dt = timing ? wall_clock64() - t_in : 0;
       if (TIMING) st[ST_INTERACT_TICKS] += dt;
@@ -706,6 +704,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           if (TIMING) st[ST_CLS_TICKS + k] += dt;
         }
     }
+    if (__ballot(L.bad != 0 || L.err != 0)) lane_report(L);
     if (++busy >= REFRESH) {  // in flight while this iteration's stores retire
       busy = 0;
       fresh = true;
@@ -770,9 +769,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           u64 *box = P.mbox + (u64)target * MBOX_WORDS;
           const u32 bot0 = lane_at(my_bot, sc);
           if (lane < give) {
-            const u32 s2 = (ring_base(sc) + ((bot0 + lane) & (ring_cap(sc) - 1))) * 2;
-            gst(box + 16 + 2 * lane, bag[s2]);
-            gst(box + 16 + 2 * lane + 1, bag[s2 + 1]);
+            const pair r = bag[ring_base(sc) + ((bot0 + lane) & (ring_cap(sc) - 1))];
+            gst(box + 16 + 2 * lane, r.a);
+            gst(box + 16 + 2 * lane + 1, r.b);
           }
           publish();
           if (lane == 0) {

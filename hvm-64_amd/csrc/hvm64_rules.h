@@ -14,6 +14,8 @@
 #define HVM_CAS(p, e, v) \
   __hip_atomic_compare_exchange_strong((p), (e), (v), __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
 #define HVM_LDS_FAA(p, v) atomicAdd((p), (v))
+// True on any lane of the wave that is running.
+#define HVM_ANY(c) (__ballot(c) != 0)
 // Pinned host memory (serving rings): system-scope accesses.
 #define HVM_LD_SYS(p) __hip_atomic_load((p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
 #define HVM_ST_SYS(p, v) __hip_atomic_store((p), (v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
@@ -21,8 +23,9 @@
 // A pointer known to address LDS (ds_* instructions, never flat ones).
 typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 #define HVM_TO_LDS(p) ((lds_u64 *)(p))
-// Retire every outstanding vector memory operation of this wave (vmcnt(0)).
-#define HVM_PUBLISH() __builtin_amdgcn_s_waitcnt(0x0F70)
+// Retire every outstanding vector memory operation of this wave (vmcnt(0));
+// no memory access moves across it.
+#define HVM_PUBLISH() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 // The same wait, placed where nothing is outstanding but loads whose results
 // are dead on some paths: it clears the compiler's record of them, which
 // would otherwise put a vmcnt wait (that also waits for the stores issued
@@ -37,6 +40,7 @@ typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 #define HVM_FAA(p, v) __atomic_fetch_add((p), (v), __ATOMIC_RELAXED)
 #define HVM_CAS(p, e, v) __atomic_compare_exchange_n((p), (e), (v), false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)
 #define HVM_LDS_FAA(p, v) __atomic_fetch_add((p), (v), __ATOMIC_RELAXED)
+#define HVM_ANY(c) (c)
 #define HVM_LD_SYS(p) __atomic_load_n((p), __ATOMIC_RELAXED)
 #define HVM_ST_SYS(p, v) __atomic_store_n((p), (v), __ATOMIC_RELAXED)
 #define HVM_FENCE_SYS() __atomic_thread_fence(__ATOMIC_RELEASE)
@@ -92,6 +96,9 @@ DEV u64 *hw(const Params &P, u64 addr) {
   return P.heap + (off >> 3);
 }
 DEV u64 ld(const Params &P, u64 addr) { return HVM_LD(hw(P, addr)); }
+struct Lane;
+// The same check for a lane's accesses (below).
+DEV u64 *hw(Lane &L, u64 addr);
 // Both words of a node (16-byte aligned) in one agent-scope store.  A store
 // ahead of a load delays that load until the store is acknowledged (the
 // vector memory counter retires in order), so a node costs one store, not
@@ -111,8 +118,6 @@ DEV void st16(u64 *p, u64 w0, u64 w1) {
   HVM_ST(p + 1, w1);
 #endif
 }
-DEV void st(const Params &P, u64 addr, u64 v) { HVM_ST(hw(P, addr), v); }
-DEV u64 xchg(const Params &P, u64 addr, u64 v) { return HVM_XCHG(hw(P, addr), v); }
 DEV u64 gld(u64 *p) { return HVM_LD(p); }
 DEV void gst(u64 *p, u64 v) { HVM_ST(p, v); }
 DEV u32 gld32(u32 *p) { return HVM_LD(p); }
@@ -127,18 +132,28 @@ DEV u64 norm_endpoint(u64 p) { return is_endpoint(p) ? (paddr(p) | T_VAR) : p; }
 // ---------------------------------------------------------------------------
 // per-lane state
 // ---------------------------------------------------------------------------
+// Two words side by side in LDS, moved by one 16-byte access.
+struct alignas(16) pair {
+  u64 a, b;
+};
+
 struct Lane {
   const Params *P;
-  // allocator: this lane's slice of its wave's ring: nodes
-  // sub_node0 + 64*i for i in [0, P->wave_nodes / 64)
-  u64 sub_node0;
-  u64 apos;            // allocations from the slice since the heap was reset
+  // allocator: this lane's slice of its wave's ring: the nodes at
+  // slice + SLICE_STRIDE*i for i in [0, slice_n)
+  u64 slice;
+  u32 slice_n;
+  u32 apos;            // allocations from the slice since the heap was reset
   u64 *apos_home;      // where apos is kept between launches
   u32 slice_rest;      // allocations left to take from the overflow ring
   u32 ov_left;         // nodes left in the current overflow run
-  u64 ov_cur;          // next overflow-ring position of that run
-  // free cache: nodes this lane consumed, newest first (fc0 .. fc{fcn-1})
-  u64 fc0, fc1, fc2, fc3;
+  u32 ov_cur;          // next overflow-ring position of that run
+  // (in_lds: the lane has redex rings and a free cache in LDS; a constant in
+  // every kernel)
+  bool in_lds;
+  // free cache: nodes this lane consumed, oldest first: FC[i * 64] for
+  // i < fcn
+  u64 *FC;
   u32 fcn;
   // arenas: the net of the running task, and the lane's chunk of an arena
   // (nodes [a_pos, a_end) of net a_net; a_net = NO_NET: none)
@@ -163,16 +178,14 @@ struct Lane {
   // looked at only at the next loop pass (acct_delta 0: none)
   u32 acct_old, acct_delta, acct_net;
   u64 a_pos, a_end;
-  bool dirty;          // stores of new nodes/cells not yet retired
-  // links deferred by the running definition: pair i at PL[2i * 64],
-  // PL[(2i + 1) * 64] (LDS; nullptr: link at once)
-  u64 *PL;
+  // links deferred by the running task: pair i at PL[i * 64] (LDS)
+  pair *PL;
   // trg registers: T[s * 64] (LDS for small definitions, else global)
   u64 *T_lds;
   u64 *T_glb;
-  // LDS redex rings, RING_PAIRS pairs (nullptr: push straight to the
-  // global ring); per-ring push counters and oldest entries
-  u64 *bag;
+  // LDS redex rings, RING_PAIRS pairs (without them redexes go straight to
+  // the global ring); per-ring push counters and oldest entries
+  pair *bag;
   u32 *bag_top;
   const u32 *bag_bot;
   // the book in LDS (nullptr: read it from global memory): definition
@@ -183,9 +196,41 @@ struct Lane {
   u32 book_ins, book_lab, book_cdef, book_tmpl;
   // counters
   u32 rw[RW_SLOTS];
+  // errors of this lane not yet reported (lane_report): the last address
+  // outside the heap (0: none), and the first other error's code and site
+  u64 bad;
+  u32 err;
 };
 
-DEV void fail(Lane &L, u32 code, u32 site = 0) { report_error(L.P->g, code, site); }
+// A lane records its errors in registers and goes on; the kernel reports
+// them when the wave's tasks have ended (lane_report).  Reporting on the
+// spot put a function call, and the register moves that a call's convention
+// asks for, behind every heap access.
+DEV void fail(Lane &L, u32 code, u32 site = 0) {
+  if (L.err == 0) L.err = code | site << 16;
+}
+
+// The word at engine address `addr`; an address outside the heap is
+// recorded and redirected to the dump words.  Selects, no branch: a branch
+// that is never taken still costs its exec-mask bookkeeping on every access.
+DEV u64 *hw(Lane &L, u64 addr) {
+  const Params &P = *L.P;
+  const u64 off = addr - HVM_HEAP_OFF;
+  const bool out = off >= P.heap_words * 8;
+  L.bad = out ? addr : L.bad;
+  return P.heap + ((out ? DUMP_WORD * 8 : off) >> 3);
+}
+DEV u64 ld(Lane &L, u64 addr) { return HVM_LD(hw(L, addr)); }
+DEV void st(Lane &L, u64 addr, u64 v) { HVM_ST(hw(L, addr), v); }
+DEV u64 xchg(Lane &L, u64 addr, u64 v) { return HVM_XCHG(hw(L, addr), v); }
+
+// Reports what the lane recorded (the first report of a launch is kept).
+DEV void lane_report(Lane &L) {
+  if (L.bad) report_error(L.P->g, ERR_BADPTR, BAD_HEAP_ADDR, L.bad);
+  if (L.err) report_error(L.P->g, L.err & 0xFFFF, L.err >> 16);
+  L.bad = 0;
+  L.err = 0;
+}
 
 // The book is read from LDS (L.book) rather than from global memory.
 DEV bool has_book(const Lane &L) { return L.lds_all || L.book != nullptr; }
@@ -210,64 +255,53 @@ DEV void count_rare(Lane &L, u32 k, u32 n) {
 // nodes (one atomic per run; a run in the overflow ring's first lap is free
 // without reads, later laps check every slot).
 static const u32 SCAN_MISSES = 8;
-static const u32 FREE_CACHE = 4;  // nodes a lane keeps for reuse (registers)
+static const u32 FREE_CACHE = 4;  // nodes a lane keeps for reuse (LDS)
 static const u32 SLICE_REST = 256;
 static const u32 OV_RUN = 64;
+static const u64 SLICE_STRIDE = 64 * 16;  // bytes between a slice's nodes
+static_assert(TSLOT_STRIDE == SLICE_STRIDE, "a template's slots are consecutive nodes of a slice");
 
-// The slow path takes and returns the cursor by value (the lane state stays
-// in registers).
-struct AllocCursor {
-  u64 apos, ov_cur;
-  u32 slice_rest, ov_left;
-  u32 misses, ov_allocs;  // counter increments
-  u64 addr;               // the node allocated (dump_addr() and err on OOM)
-  u32 err;
-};
-
-// Ring slots are in the heap by construction of the layout (no bounds check).
-NOINL AllocCursor alloc_slow(u64 *heap, Globals *g, u64 wave_nodes, u64 ov_node0, u64 ov_nodes, u64 sub_node0,
-                             AllocCursor c) {
-  const u64 n = wave_nodes / 64;
-  c.err = 0;
-  if (c.slice_rest == 0) {
+// One node past the slice's first lap (the free cache is empty).  Ring slots
+// are in the heap by construction of the layout (no bounds check).
+DEV u64 alloc_lapped(Lane &L) {
+  const Params &P = *L.P;
+  u64 *const heap = P.heap;
+  if (L.slice_rest == 0) {
     for (u32 miss = 0; miss < SCAN_MISSES; miss++) {
-      u64 node = sub_node0 + (c.apos % n) * 64;
-      c.apos++;
-      u64 w0 = HVM_LD(heap + 2 * node), w1 = HVM_LD(heap + 2 * node + 1);
-      if (w0 == P_FREE && w1 == P_FREE) {
-        c.addr = HVM_HEAP_OFF + node * 16;
-        return c;
+      const u64 addr = L.slice + (u64)(L.apos % L.slice_n) * SLICE_STRIDE;
+      if (++L.apos >= 1u << 31) {  // keep the position within 32 bits (the allocation count stays exact)
+        const u32 whole = L.apos / L.slice_n * L.slice_n - L.slice_n;
+        L.apos -= whole;
+        count_rare(L, RW_REUSE, whole);
       }
-      c.misses++;
+      u64 *w = heap + ((addr - HVM_HEAP_OFF) >> 3);
+      const u64 w0 = HVM_LD(w), w1 = HVM_LD(w + 1);
+      if (w0 == P_FREE && w1 == P_FREE) return addr;
+      count_rare(L, RW_ALLOC_MISS, 1);
     }
-    c.slice_rest = SLICE_REST;
+    L.slice_rest = SLICE_REST;
   } else {
-    c.slice_rest--;
+    L.slice_rest--;
   }
-  c.ov_allocs++;
+  count_rare(L, RW_OV_ALLOC, 1);
   // Overflow slots are shared: a slot is taken by swapping its first word
   // from FREE (so two lanes whose runs alias the same slot a lap apart can
   // never both take it), and kept only if its second word is FREE too.
-  for (u64 miss = 0; miss <= ov_nodes; miss++) {
-    if (c.ov_left == 0) {
-      c.ov_cur = HVM_FAA(&g->ov_pos, (u64)OV_RUN);
-      c.ov_left = OV_RUN;
+  for (u64 miss = 0; miss <= P.ov_nodes; miss++) {
+    if (L.ov_left == 0) {
+      L.ov_cur = (u32)HVM_FAA(&P.g->ov_pos, (u64)OV_RUN);
+      L.ov_left = OV_RUN;
     }
-    u64 pos = c.ov_cur++;
-    c.ov_left--;
-    u64 node = ov_node0 + (pos & (ov_nodes - 1));
+    const u64 node = P.ov_node0 + (L.ov_cur++ & (P.ov_nodes - 1));
+    L.ov_left--;
     u64 expect = P_FREE;
     if (HVM_CAS(heap + 2 * node, &expect, P_NONE)) {
-      if (HVM_LD(heap + 2 * node + 1) == P_FREE) {
-        c.addr = HVM_HEAP_OFF + node * 16;
-        return c;
-      }
+      if (HVM_LD(heap + 2 * node + 1) == P_FREE) return HVM_HEAP_OFF + node * 16;
       HVM_ST(heap + 2 * node, P_FREE);  // second word in use: not a free node
     }
   }
-  c.err = ERR_OOM;
-  c.addr = dump_addr();
-  return c;
+  fail(L, ERR_OOM);
+  return dump_addr();
 }
 
 // Per-net arenas.  Net i's arena is a list of extents: its initial extent
@@ -299,9 +333,7 @@ DEV u64 refill_of(u64 len, u64 max_refill) {
   return h < ARENA_MIN_REFILL ? ARENA_MIN_REFILL : h > max_refill ? max_refill : h;
 }
 
-// Out of line, with plain arguments: a reference to the kernel's Params
-// would make the compiler copy them to scratch memory.
-NOINL ArenaChunk arena_take(u64 *word, u64 base0, u64 len0, u64 max_refill, u32 gs, u64 *pool_next, u64 pool_end,
+DEV ArenaChunk arena_take(u64 *word, u64 base0, u64 len0, u64 max_refill, u32 gs, u64 *pool_next, u64 pool_end,
                             u32 *gmap, u32 net, u64 *ov_next, u64 ov_end, u32 n) {
   ArenaChunk c;
   c.err = 0;
@@ -388,44 +420,62 @@ DEV void arena_room(Lane &L, u32 need) {
   }
 }
 
-DEV u64 alloc_node(Lane &L) {
+// `need` (at most N) nodes: out[0 .. need).  From the free cache, newest
+// first, then from the slice's first lap; both are address arithmetic
+// without a branch.  Past the first lap one by one, in a loop, so that the
+// scan is in the code once per call site.
+template <u32 N>
+DEV void alloc_nodes(Lane &L, u32 need, u64 (&out)[N]) {
   if (L.arenas) {
-    arena_room(L, 1);
-    return L.a_pos < L.a_end ? HVM_HEAP_OFF + (L.a_pos++) * 16 : dump_addr();
+    if (need) arena_room(L, need);
+    const bool ok = L.a_pos + need <= L.a_end;
+#pragma unroll
+    for (u32 j = 0; j < N; j++) out[j] = ok ? HVM_HEAP_OFF + (L.a_pos + j) * 16 : dump_addr();
+    L.a_pos += ok ? need : 0;
+    return;
   }
-  if (L.fcn) {
-    const u64 a = L.fc0;
-    L.fc0 = L.fc1;
-    L.fc1 = L.fc2;
-    L.fc2 = L.fc3;
-    L.fcn--;
-    L.rw[RW_REUSE]++;
-    return a;
+  const u32 used = L.in_lds ? (L.fcn < need ? L.fcn : need) : 0;
+  const u32 apos = L.apos + need - used;
+  if (need > used && apos > L.slice_n) {
+    for (u32 j = 0; j < need; j++) {
+      u64 v;
+      if (L.in_lds && L.fcn) {
+        v = L.FC[--L.fcn * 64];
+        L.rw[RW_REUSE]++;
+      } else if (L.apos < L.slice_n) {
+        v = L.slice + (u64)L.apos++ * SLICE_STRIDE;
+      } else {
+        v = alloc_lapped(L);
+      }
+#pragma unroll
+      for (u32 k = 0; k < N; k++) out[k] = k == j ? v : out[k];
+    }
+    return;
   }
-  const u64 n = L.P->wave_nodes / 64;
-  if (L.apos < n) return HVM_HEAP_OFF + (L.sub_node0 + (L.apos++) * 64) * 16;
-  AllocCursor c;
-  c.apos = L.apos;
-  c.ov_cur = L.ov_cur;
-  c.slice_rest = L.slice_rest;
-  c.ov_left = L.ov_left;
-  c.misses = 0;
-  c.ov_allocs = 0;
-  const Params &P = *L.P;
-  c = alloc_slow(P.heap, P.g, P.wave_nodes, P.ov_node0, P.ov_nodes, L.sub_node0, c);
-  L.apos = c.apos;
-  L.ov_cur = c.ov_cur;
-  L.slice_rest = c.slice_rest;
-  L.ov_left = c.ov_left;
-  count_rare(L, RW_ALLOC_MISS, c.misses);
-  count_rare(L, RW_OV_ALLOC, c.ov_allocs);
-  if (c.err) fail(L, c.err);
-  return c.addr;
+#pragma unroll
+  for (u32 j = 0; j < N; j++) {
+    const u64 fresh = L.slice + (u64)(L.apos + j - used) * SLICE_STRIDE;
+    if (L.in_lds && j < FREE_CACHE) {
+      const u64 cached = L.FC[(j < used ? L.fcn - 1 - j : 0) * 64];
+      out[j] = j < used ? cached : fresh;
+    } else {
+      out[j] = fresh;
+    }
+  }
+  L.apos = apos;
+  if (L.in_lds) L.fcn -= used;
+  L.rw[RW_REUSE] += used;
+}
+
+DEV u64 alloc_node(Lane &L) {
+  u64 n[1];
+  alloc_nodes(L, 1, n);
+  return n[0];
 }
 
 // Two node words.  Agent-scope stores: a plain store may stay in the
 // writing XCD's L2, where lanes on the other XCDs would not see it.
-DEV void st2(const Params &P, u64 addr, u64 w0, u64 w1) { st16(hw(P, addr), w0, w1); }
+DEV void st2(Lane &L, u64 addr, u64 w0, u64 w1) { st16(hw(L, addr), w0, w1); }
 
 // Both words of a published node (immutable until taken) in one 16-byte
 // agent-scope load; two nodes: two loads and one wait.  The compiler does not
@@ -465,24 +515,24 @@ DEV void ld16(const u64 *p, u64 &p0, u64 &p1) {
 // A fresh pair of var cells (both words of one node): cells n and n + 8.
 DEV u64 alloc_vars2(Lane &L) {
   u64 n = alloc_node(L);
-  st2(*L.P, n, P_NONE, P_NONE);
-  L.dirty = true;
+  st2(L, n, P_NONE, P_NONE);
   return n;
 }
 
 // One fresh var cell; the node's other word stays FREE.
 DEV u64 alloc_var1(Lane &L) {
   u64 n = alloc_node(L);
-  st2(*L.P, n, P_NONE, P_FREE);
-  L.dirty = true;
+  st2(L, n, P_NONE, P_FREE);
   return n;
 }
 
-DEV u64 new_node(Lane &L, u32 tag, u32 lab, u64 p1, u64 p2) {
-  u64 n = alloc_node(L);
-  st2(*L.P, n, norm_endpoint(p1), norm_endpoint(p2));
-  L.dirty = true;
-  return mkport(tag, lab, n);
+// Two words of a node this lane has just allocated (always in the heap).
+DEV void st2_new(const Params &P, u64 addr, u64 w0, u64 w1) {
+  st16(P.heap + ((addr - HVM_HEAP_OFF) >> 3), w0, w1);
+}
+// The same for a node's aux ports.
+DEV void node_new(const Params &P, u64 addr, u64 p1, u64 p2) {
+  st2_new(P, addr, norm_endpoint(p1), norm_endpoint(p2));
 }
 
 // A node this lane has consumed (its words already read).  Per-net arenas
@@ -493,12 +543,8 @@ DEV u64 new_node(Lane &L, u32 tag, u32 lab, u64 p1, u64 p2) {
 DEV void drop_node(Lane &L, u64 *w) {
   if (L.arenas) return;
   const u64 off = (u64)(w - L.P->heap);
-  if (L.fcn < FREE_CACHE && off >= RESERVED_WORDS) {
-    L.fc3 = L.fc2;
-    L.fc2 = L.fc1;
-    L.fc1 = L.fc0;
-    L.fc0 = HVM_HEAP_OFF + off * 8;
-    L.fcn++;
+  if (L.in_lds && L.fcn < FREE_CACHE && off >= RESERVED_WORDS) {
+    L.FC[L.fcn++ * 64] = HVM_HEAP_OFF + off * 8;
     return;
   }
   st16(w, P_FREE, P_FREE);
@@ -507,14 +553,14 @@ DEV void drop_node(Lane &L, u64 *w) {
 // Consume a binary node: read both aux words, then drop the node.
 DEV void take(Lane &L, u64 p, u64 &x, u64 &y) {
   u64 a = paddr(p);
-  u64 *w = hw(*L.P, a & ~15ull);
+  u64 *w = hw(L, a & ~15ull);
   ld16(w, x, y);
   drop_node(L, w);
 }
 
 // take() of two nodes, their loads in flight together.
 DEV void take2(Lane &L, u64 p, u64 q, u64 &p1, u64 &p2, u64 &q1, u64 &q2) {
-  u64 *wp = hw(*L.P, paddr(p) & ~15ull), *wq = hw(*L.P, paddr(q) & ~15ull);
+  u64 *wp = hw(L, paddr(p) & ~15ull), *wq = hw(L, paddr(q) & ~15ull);
   ld16x2(wp, wq, p1, p2, q1, q2);
   drop_node(L, wp);
   drop_node(L, wq);
@@ -523,22 +569,14 @@ DEV void take2(Lane &L, u64 p, u64 q, u64 &p1, u64 &p2, u64 &q1, u64 &q2) {
 // A var cell both of whose sides have arrived: marked FREE for the ring scan
 // (arenas never reuse it).
 DEV void free_cell(Lane &L, u64 c) {
-  if (!L.arenas) st(*L.P, c, P_FREE);
-}
-
-// Retire this lane's stores before a port to new memory becomes visible.
-DEV void publish_if_dirty(Lane &L) {
-  if (L.dirty) {
-    publish();
-    L.dirty = false;
-  }
+  if (!L.arenas) st(L, c, P_FREE);
 }
 
 // ---------------------------------------------------------------------------
 // redexes
 // ---------------------------------------------------------------------------
 // Push one redex to the global ring (retires the lane's stores first).
-NOINL void push_global(u64 *queue, u64 qmask, Globals *g, u64 a, u64 b) {
+DEV void push_global(u64 *queue, u64 qmask, Globals *g, u64 a, u64 b) {
   publish();
   u64 pos = HVM_FAA(&g->q_tail, 1ull);
   u64 *s = queue + (pos & qmask) * 2;
@@ -554,41 +592,39 @@ DEV void global_push1(Lane &L, u64 a, u64 b) {
   // wave before this task ends, so it is counted for its net at once
   if (L.serve) HVM_FAA(&L.P->pending[L.cur_net], 1u);
   push_global(L.P->queue, L.P->qmask, L.P->g, a, b);
-  L.dirty = false;
 }
 
-// The rule a redex will take, grouped: the arms of interact() that run
+// The rule a redex will take, grouped: the arms of interact.rs:6-44 that run
 // anni2, comm22, a definition call (a non-ERA Ref), and everything else.
 // Calls go to the ring of the definition's group (DefRec::group, by
 // instruction count), read from the book in LDS; a wave runs one call ring
 // per iteration and waits for its longest definition, so definitions of
 // similar length share a ring.  Without the LDS book: definition modulo NCALL.
+// An ExpandDef (a Ref to a heap cell) goes to the first.
+// No branches: the redexes of a wave's lanes are of all kinds.
 DEV u32 redex_class(u64 a, u64 b, const lds_u64 *book, bool lds, u32 ndefs) {
-  u32 at = ptag(a), bt = ptag(b);
-  const bool aref = at == T_REF && a != P_ERA, bref = bt == T_REF && b != P_ERA;
-  if (aref || bref) {
-    const u64 addr = paddr(aref ? a : b);
-    if (addr_in_heap(addr)) return CLS_CALL;
-    const u32 di = def_index(addr);
-    const u32 g = lds ? (di < ndefs ? (u32)book[4 * di + 3] : 0u) : di;
-    return CLS_CALL + g % NCALL;
-  }
-  if (at == bt) {
-    if (at == T_OP || at == T_SWI) return CLS_ANNI;
-    if (at == T_CTR) return plab(a) == plab(b) ? CLS_ANNI : CLS_COMM;
-    return CLS_OTHER;
-  }
-  if ((at == T_CTR && bt == T_OP) || (at == T_OP && bt == T_CTR)) return CLS_COMM;
-  if ((at == T_CTR && bt == T_SWI && plab(a) != 0) || (at == T_SWI && bt == T_CTR && plab(b) != 0)) return CLS_COMM;
-  return CLS_OTHER;
+  const u32 at = ptag(a), bt = ptag(b), la = plab(a), lb = plab(b);
+  const bool aref = (at == T_REF) & (a != P_ERA), bref = (bt == T_REF) & (b != P_ERA);
+  const u64 r = aref ? a : b;
+  const bool call = aref | bref, heap = addr_in_heap(paddr(r));
+  const u32 di = def_index((u64)(u32)paddr(r));
+  u32 g;
+  if (lds) g = (u32)book[4 * ((call & !heap & (di < ndefs)) ? di : 0u) + 3];
+  else g = di;
+  g = heap ? 0u : g % NCALL;
+  const bool same = (at == bt) & (at >= T_OP), ctrs = same & (at == T_CTR);
+  const bool anni = same & (!ctrs | (la == lb));
+  const bool op_ctr = (at ^ bt) == (T_CTR ^ T_OP) && (at == T_CTR || bt == T_CTR);
+  const bool swi_ctr = (at ^ bt) == (T_CTR ^ T_SWI) && (at == T_CTR || bt == T_CTR);
+  const bool comm = (ctrs & (la != lb)) | op_ctr | (swi_ctr & ((at == T_CTR ? la : lb) != 0));
+  return call ? CLS_CALL + g : anni ? CLS_ANNI : comm ? CLS_COMM : CLS_OTHER;
 }
 
 // linker.rs:70-85: skippable pairs count as an erasure and are dropped.
 DEV void redux(Lane &L, u64 a, u64 b) {
-  if (is_skippable(a) && is_skippable(b)) {
-    L.rw[RW_ERAS]++;
-    return;
-  }
+  const bool skip = is_skippable(a) & is_skippable(b);
+  L.rw[RW_ERAS] += skip;
+  if (skip) return;
   if (L.serve) {
     if (!reaches_heap(a) && !reaches_heap(b)) {  // no net to count it for: run it in this task
       if (L.inl_n >= SERVE_INL) {
@@ -601,13 +637,11 @@ DEV void redux(Lane &L, u64 a, u64 b) {
       return;
     }
   }
-  if (L.bag) {
-    u32 c = redex_class(a, b, L.book, has_book(L), L.P->ndefs);
-    u32 idx = HVM_LDS_FAA(&L.bag_top[c], 1u);
+  if (L.in_lds) {
+    const u32 c = redex_class(a, b, L.book, has_book(L), L.P->ndefs);
+    const u32 idx = HVM_LDS_FAA(&L.bag_top[c], 1u);
     if (idx - L.bag_bot[c] < ring_cap(c)) {
-      u32 k = (ring_base(c) + (idx & (ring_cap(c) - 1))) * 2;
-      L.bag[k] = a;
-      L.bag[k + 1] = b;
+      L.bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
       if (L.serve) L.pushed++;  // counted when the task ends (a full ring's redex is counted at once, below)
       return;
     }
@@ -620,7 +654,7 @@ DEV void redux(Lane &L, u64 a, u64 b) {
 // its port there; the second finds it, frees the cell and links on.
 //
 // Rules never link directly: they append (a, b) pairs to the lane's link
-// list (LDS, LINK_CAP pairs), and the lane's task loop (run_task) links the
+// list (LDS, LINK_CAP pairs), and its task loop (run_tasks, run_def) links the
 // whole list at one place in the code, four swaps in flight at a time.  A
 // swap that finds the other endpoint's port frees the cell and appends the
 // continuation link to the list.  Every continuation consumes a var cell, so
@@ -630,85 +664,112 @@ static const u32 MAX_CHAIN = 1u << 24;
 // Every producer checks the room it needs (interp_run: one link per
 // instruction; a rule: at most four, into an empty list).
 DEV void push_link(Lane &L, u32 &np, u64 a, u64 b) {
-  L.PL[(u64)(2 * np) * 64] = a;
-  L.PL[(u64)(2 * np + 1) * 64] = b;
+  L.PL[np * 64] = pair{a, b};
   np++;
 }
 
-// First step of one link: true with `cell` set when a swap of
-// norm_endpoint(b) into `cell` is due, false when the link is complete.
-DEV bool link_begin(Lane &L, u64 &a, u64 &b, u64 &cell) {
-  if (!is_endpoint(a)) {
-    if (!is_endpoint(b)) {
-      redux(L, a, b);
-      return false;
-    }
-    u64 t = a;
-    a = b;
-    b = t;
-  }
-  cell = paddr(a);
-  return true;
-}
-
-// Links every pair of the list (the list is empty afterwards).
+// Links every pair of the list (the list is empty afterwards), four at a
+// time: a pair of principal ports is a redex; the others swap their value
+// into the endpoint's cell, the (up to) four swaps in flight together.
+// The redexes go to the rings while the stores of new nodes retire, in as
+// many passes as the lane with the most of them has.
 DEV void flush_links(Lane &L, u32 &np) {
-  const Params &P = *L.P;
-  u64 *PL = L.PL;
   for (u32 round = 0; np > 0; round++) {
     if (round > MAX_CHAIN) {
       fail(L, ERR_BADPTR, BAD_CHAIN);
       np = 0;
       return;
     }
-    // take the last (up to) four pairs
     const u32 cnt = np < 4 ? np : 4;
     np -= cnt;
-    u64 a[4], b[4], c[4], o[4];
-    bool p[4];
+    pair p[4];
+    u32 red = 0, cell = 0;  // bit j: pair j is a redex / swaps
+#pragma unroll
+    for (u32 j = 0; j < 4; j++) p[j] = L.PL[(np + j) * 64];  // np + j < LINK_CAP: np > 0 only when cnt == 4
 #pragma unroll
     for (u32 j = 0; j < 4; j++) {
-      a[j] = j < cnt ? PL[(u64)(2 * (np + j)) * 64] : 0;
-      b[j] = j < cnt ? PL[(u64)(2 * (np + j) + 1) * 64] : 0;
-      c[j] = 0;
+      // the endpoint (if there is one) to `a`
+      const bool ea = is_endpoint(p[j].a), eb = is_endpoint(p[j].b), in = j < cnt;
+      const u64 a = ea ? p[j].a : p[j].b, b = ea ? p[j].b : p[j].a;
+      red |= (in & !ea & !eb) ? 1u << j : 0u;
+      cell |= (in & (ea | eb)) ? 1u << j : 0u;
+      p[j].a = a;
+      p[j].b = b;
     }
+    while (red) {
+      // (a redex's two sides were exchanged above: exchange them back)
+      u64 a = p[3].b, b = p[3].a;
 #pragma unroll
-    for (u32 j = 0; j < 4; j++) p[j] = j < cnt && link_begin(L, a[j], b[j], c[j]);
-    if (p[0] || p[1] || p[2] || p[3]) publish_if_dirty(L);
+      for (u32 j = 3; j-- > 0;) {
+        const bool here = (red >> j) & 1;
+        a = here ? p[j].b : a;
+        b = here ? p[j].a : b;
+      }
+      red &= red - 1;
+      redux(L, a, b);
+    }
+    publish();
+    u64 o[4];
 #pragma unroll
-    for (u32 j = 0; j < 4; j++) o[j] = p[j] ? xchg(P, c[j], norm_endpoint(b[j])) : P_NONE;
+    for (u32 j = 0; j < 4; j++) {
+      u64 *const w = hw(L, (cell >> j) & 1 ? paddr(p[j].a) : dump_addr());
+      o[j] = P_NONE;
+      if ((cell >> j) & 1) o[j] = HVM_XCHG(w, norm_endpoint(p[j].b));
+      p[j].a = paddr(p[j].a);
+    }
 #pragma unroll
     for (u32 j = 0; j < 4; j++) {
       if (o[j] != P_NONE) {  // second arrival: free the cell, link on
-        free_cell(L, c[j]);
-        PL[(u64)(2 * np) * 64] = o[j];
-        PL[(u64)(2 * np + 1) * 64] = b[j];
-        np++;
+        free_cell(L, p[j].a);
+        push_link(L, np, o[j], p[j].b);
       }
     }
   }
 }
 
 // Follow a wire endpoint whose other side has already linked (the
-// reference's Trg::target on a wire, linker.rs:278-280).  The caller owns the
-// endpoint, so once a cell holds a port the cell is ours to free.
-DEV u64 resolve(Lane &L, u64 p) {
-  const Params &P = *L.P;
-  for (u32 hop = 0; is_endpoint(p); hop++) {
+// reference's Trg::target on a wire, linker.rs:278-280), when `go`.  The
+// caller owns the endpoint, so once a cell holds a port the cell is ours to
+// free.
+DEV u64 follow(Lane &L, u64 p, bool go) {
+  for (u32 hop = 0; go; hop++) {
     if (hop > MAX_CHAIN) {
       fail(L, ERR_BADPTR, BAD_RESOLVE);
       return P_ERA;
     }
-    u64 c = paddr(p);
-    u64 v = ld(P, c);
-    if (v == P_NONE) break;
-    free_cell(L, c);
-    p = v;
+    u64 *const w = hw(L, paddr(p));
+    const u64 v = HVM_LD(w);
+    go = v != P_NONE;
+    if (go) {
+      if (!L.arenas) HVM_ST(w, P_FREE);
+      p = v;
+      go = is_endpoint(v);
+    }
   }
   return p;
 }
+DEV u64 resolve(Lane &L, u64 p) { return follow(L, p, is_endpoint(p)); }
 
 DEV u64 as_wire(u64 p) { return is_endpoint(p) ? wire_port(paddr(p)) : p; }
+
+// operate_binary, whose unsigned operations that neither divide nor shift
+// are computed here: they are nearly all of a program's, and the general
+// function is a call (and a second one inside), with its result by memory.
+DEV u32 num_binary(Lane &L, u32 a, u32 op, u32 b) {
+  const u32 p = num_u24(a), q = num_u24(b);
+  u32 r = op == N_ADD ? p + q : op == N_SUB ? p - q : op == N_SUBS ? q - p : op == N_MUL ? p * q
+          : op == N_EQ ? (u32)(p == q) : op == N_NE ? (u32)(p != q) : op == N_LT ? (u32)(p < q)
+          : op == N_GT ? (u32)(p > q) : op == N_AND ? (p & q) : op == N_OR ? (p | q) : (p ^ q);
+  const u32 fast = 1u << N_ADD | 1u << N_SUB | 1u << N_SUBS | 1u << N_MUL | 1u << N_EQ | 1u << N_NE | 1u << N_LT |
+                   1u << N_GT | 1u << N_AND | 1u << N_OR | 1u << N_XOR;
+  u32 out = num_new_u24(r);
+  if (num_tag(a) != N_U24 || num_tag(b) != N_U24 || op >= N_TAGS || !((fast >> op) & 1)) {
+    bool div0 = false;
+    out = operate_binary(a, op, b, &div0);
+    if (div0) fail(L, ERR_DIV0);
+  }
+  return out;
+}
 
 // ---------------------------------------------------------------------------
 // interaction rules (interact.rs); each appends at most 4 links
@@ -722,20 +783,23 @@ DEV void anni2(Lane &L, u32 &np, u64 a, u64 b) {
 }
 
 DEV void comm22(Lane &L, u32 &np, u64 a, u64 b) {
+  const Params &P = *L.P;
   L.rw[RW_COMM]++;
   u64 a1, a2, b1, b2;
   take2(L, a, b, a1, a2, b1, b2);
-  if (L.arenas) arena_room(L, 6);  // the six nodes below, in one take
-  u64 v1 = alloc_vars2(L), v3 = alloc_vars2(L);
-  u64 v2 = v1 + 8, v4 = v3 + 8;
-  u64 A1 = new_node(L, ptag(a), plab(a), var_port(v1), var_port(v2));
-  u64 A2 = new_node(L, ptag(a), plab(a), var_port(v3), var_port(v4));
-  u64 B1 = new_node(L, ptag(b), plab(b), var_port(v1), var_port(v3));
-  u64 B2 = new_node(L, ptag(b), plab(b), var_port(v2), var_port(v4));
-  push_link(L, np, a1, B1);
-  push_link(L, np, a2, B2);
-  push_link(L, np, b1, A1);
-  push_link(L, np, b2, A2);
+  u64 n[6];
+  alloc_nodes(L, 6, n);
+  const u64 v1 = var_port(n[0]), v2 = var_port(n[0] + 8), v3 = var_port(n[1]), v4 = var_port(n[1] + 8);
+  st2_new(P, n[0], P_NONE, P_NONE);
+  st2_new(P, n[1], P_NONE, P_NONE);
+  st2_new(P, n[2], v1, v2);
+  st2_new(P, n[3], v3, v4);
+  st2_new(P, n[4], v1, v3);
+  st2_new(P, n[5], v2, v4);
+  push_link(L, np, a1, mkport(ptag(b), plab(b), n[4]));
+  push_link(L, np, a2, mkport(ptag(b), plab(b), n[5]));
+  push_link(L, np, b1, mkport(ptag(a), plab(a), n[2]));
+  push_link(L, np, b2, mkport(ptag(a), plab(a), n[3]));
 }
 
 DEV void comm02(Lane &L, u32 &np, u64 a, u64 b) {
@@ -746,36 +810,54 @@ DEV void comm02(Lane &L, u32 &np, u64 a, u64 b) {
   push_link(L, np, b2, a);
 }
 
-DEV void switch_num(Lane &L, u32 &np, u64 a, u64 b) {  // interact.rs:201-223
-  L.rw[RW_OPER]++;
-  u64 a1, a2;
-  take(L, a, a1, a2);
-  u32 n = pnum(b);
-  u32 v = num_tag(n) == N_U24 ? num_u24(n) : 0;
-  u64 x;
-  if (v == 0) {
-    x = new_node(L, T_CTR, 0, a2, P_ERA);
-  } else {
-    u64 y = new_node(L, T_CTR, 0, numport(num_new_u24(v - 1)), a2);
-    x = new_node(L, T_CTR, 0, P_ERA, y);
+// The redexes of CLS_OTHER (the arms of interact.rs:6-44 that are neither
+// an annihilation, a comm22 nor a call): an eraser or a number meeting a
+// node.  One node is read, whichever the rule; a number meeting a Ctr, and
+// an eraser, are copied onto both aux ports (comm02, interact.rs:162-168).
+DEV void rule_other(Lane &L, u32 &np, u64 a, u64 b) {
+  const Params &P = *L.P;
+  const bool bin_a = is_binary(a);
+  const u64 y = bin_a ? a : b, n = bin_a ? b : a;  // the node, the nilary port
+  const u32 yt = ptag(y), nt = ptag(n);
+  if (!is_binary(y) || is_endpoint(y)) {
+    if (is_principal(a) && is_principal(b)) L.rw[RW_ERAS]++;
+    else fail(L, ERR_UNIMPL);
+    return;
   }
-  push_link(L, np, a1, x);
-}
-
-DEV void op_num(Lane &L, u32 &np, u64 a, u64 b) {  // interact.rs:251-270
-  u32 op = plab(a);
-  u64 a1, a2;
-  take(L, a, a1, a2);
-  a1 = resolve(L, a1);
-  if (ptag(a1) == T_NUM) {
-    L.rw[RW_OPER]++;
-    bool div0 = false;
-    u32 out = operate_binary(pnum(b), op, pnum(a1), &div0);
-    if (div0) fail(L, ERR_DIV0);
-    push_link(L, np, a2, numport(out));
+  const bool copy = n == P_ERA || (nt == T_NUM && yt == T_CTR);
+  const bool oper = nt == T_NUM && yt == T_OP, swi = nt == T_NUM && yt == T_SWI;
+  if (!(copy || oper || swi)) {  // Switch-Ctr(0), Op-Switch: unimplemented!() in the reference
+    fail(L, ERR_UNIMPL);
+    return;
+  }
+  u64 y1, y2;
+  take(L, y, y1, y2);
+  L.rw[RW_COMM] += copy;
+  const u32 num = pnum(n);
+  // op_num (interact.rs:251-270): the node's operand, when it has arrived
+  y1 = follow(L, y1, oper && is_endpoint(y1));
+  const bool done = oper && ptag(y1) == T_NUM;  // both operands: the result
+  // switch_num (interact.rs:201-223)
+  const u32 v = num_tag(num) == N_U24 ? num_u24(num) : 0;
+  L.rw[RW_OPER] += done || swi;
+  u64 m[2];
+  const u32 need = swi ? (v ? 2u : 1u) : oper && !done ? 1u : 0u;
+  if (need) alloc_nodes(L, need, m);
+  if (copy) {
+    push_link(L, np, y1, n);
+    push_link(L, np, y2, n);
+  } else if (swi) {
+    if (v == 0) node_new(P, m[0], y2, P_ERA);
+    else {
+      node_new(P, m[1], numport(num_new_u24(v - 1)), y2);
+      node_new(P, m[0], P_ERA, mkport(T_CTR, 0, m[1]));
+    }
+    push_link(L, np, y1, mkport(T_CTR, 0, m[0]));
+  } else if (done) {
+    push_link(L, np, y2, numport(num_binary(L, num, plab(y), pnum(y1))));
   } else {
-    u64 x = new_node(L, T_OP, N_SYM, numport(operate_unary(op, pnum(b))), a2);
-    push_link(L, np, a1, x);
+    node_new(P, m[0], numport(operate_unary(plab(y), num)), y2);
+    push_link(L, np, y1, mkport(T_OP, N_SYM, m[0]));
   }
 }
 
@@ -842,108 +924,72 @@ DEV void t_set(Interp &I, u32 s, u64 v) {
   else I.Tg[(u64)s * 64] = v;
 }
 
-// Two words of a node this lane has just allocated (always in the heap).
-DEV void st2_new(const Params &P, u64 addr, u64 w0, u64 w1) {
-  st16(P.heap + ((addr - HVM_HEAP_OFF) >> 3), w0, w1);
+// The instruction kinds other than Ctr that read a trg or make registers
+// (instruction.rs:134-203), and the nodes each takes with its operand `p`.
+DEV u32 other_need(u32 kind, u64 p) {
+  if (kind == I_WIRES) return 1;
+  if (kind == I_CONST || p == P_ERA) return 0;
+  if (ptag(p) != T_NUM) return 2;
+  if (kind == I_OPNUM) return 0;
+  if (kind == I_OP) return 2;
+  return num_tag(pnum(p)) == N_U24 && num_u24(pnum(p)) != 0 ? 3 : 2;  // I_SWITCH
 }
 
-// Two fresh nodes: consecutive slice positions on the first lap.
-DEV void alloc2(Lane &L, u64 &n0, u64 &n1) {
-  if (!L.arenas && L.fcn == 0 && L.apos + 2 <= L.P->wave_nodes / 64) {
-    n0 = HVM_HEAP_OFF + (L.sub_node0 + L.apos * 64) * 16;
-    n1 = n0 + 64 * 16;
-    L.apos += 2;
-    return;
-  }
-  n0 = alloc_node(L);
-  n1 = alloc_node(L);
-}
-
-// The rare instruction kinds (Op, OpNum, Switch; instruction.rs:134-203).
-DEV void exec_num(Lane &L, Interp &I, u32 kind, u32 b, u32 c, u64 w1, u64 port, u32 &np) {
+// `m`: the nodes other_need asked for.
+DEV void exec_other(Lane &L, Interp &I, u64 w0, u64 w1, u64 p, const u64 (&m)[3], u32 &np) {
   const Params &P = *L.P;
-  const u32 lab = (u32)(w1 & 0xFFFF);
-  if (kind == I_OPNUM) {  // instruction.rs:154-172
+  const u32 kind = (u32)(w0 & 0xFF), lab = (u32)(w1 & 0xFFFF);
+  const u32 a = (u32)(w0 >> 16) & 0xFFFF, b = (u32)(w0 >> 32) & 0xFFFF, c = (u32)(w0 >> 48);
+  if (kind == I_CONST) {
+    t_set(I, a, w1);
+    return;
+  }
+  if (kind == I_WIRES) {
+    st2_new(P, m[0], P_NONE, P_NONE);
+    t_set(I, a, var_port(m[0]));
+    t_set(I, b, wire_port(m[0]));
+    t_set(I, c, var_port(m[0] + 8));
+    t_set(I, lab, wire_port(m[0] + 8));
+    return;
+  }
+  const bool num = ptag(p) == T_NUM, one = kind == I_OPNUM;  // one: a single result, in c
+  const u32 n = pnum(p);
+  u64 rb, rc;
+  if (p == P_ERA) {
+    count_rare(L, kind == I_OP ? SC_OP_ERA : one ? SC_OPNUM_ERA : SC_SWITCH_ERA, 1);
+    L.rw[RW_ERAS] += kind == I_SWITCH;
+    rb = rc = P_ERA;
+  } else if (!num) {  // a node of the instruction's kind, linked to the operand
     const u32 rhs = (u32)(w1 >> 32);
-    if (ptag(port) == T_NUM) {
-      L.rw[RW_OPER]++;
-      bool div0 = false;
-      const u32 out = operate_binary(pnum(port), lab, rhs, &div0);
-      if (div0) fail(L, ERR_DIV0);
-      t_set(I, c, numport(out));
-    } else if (port == P_ERA) {
-      count_rare(L, SC_OPNUM_ERA, 1);
-      t_set(I, c, P_ERA);
-    } else {
-      u64 v, n;
-      alloc2(L, v, n);
-      st2_new(P, v, P_NONE, P_FREE);
-      st2_new(P, n, numport(rhs), var_port(v));
-      L.dirty = true;
-      push_link(L, np, port, mkport(T_OP, lab, n));
-      t_set(I, c, var_port(v));
-    }
-    return;
-  }
-  if (kind == I_OP) {  // instruction.rs:134-152
-    if (ptag(port) == T_NUM) {
-      u64 v, n;
-      alloc2(L, v, n);
-      st2_new(P, v, P_NONE, P_FREE);
-      st2_new(P, n, numport(operate_unary(lab, pnum(port))), var_port(v));
-      L.dirty = true;
-      t_set(I, b, mkport(T_OP, N_SYM, n));
-      t_set(I, c, var_port(v));
-    } else if (port == P_ERA) {
-      count_rare(L, SC_OP_ERA, 1);
-      t_set(I, b, P_ERA);
-      t_set(I, c, P_ERA);
-    } else {
-      u64 v, n;
-      alloc2(L, v, n);
-      st2_new(P, v, P_NONE, P_NONE);
-      st2_new(P, n, var_port(v), var_port(v + 8));
-      L.dirty = true;
-      push_link(L, np, port, mkport(T_OP, lab, n));
-      t_set(I, b, var_port(v));
-      t_set(I, c, var_port(v + 8));
-    }
-    return;
-  }
-  // I_SWITCH, instruction.rs:174-203
-  if (ptag(port) == T_NUM) {
+    st2_new(P, m[0], P_NONE, one ? P_FREE : P_NONE);
+    st2_new(P, m[1], one ? numport(rhs) : var_port(m[0]), one ? var_port(m[0]) : var_port(m[0] + 8));
+    push_link(L, np, p, kind == I_SWITCH ? mkport(T_SWI, 0, m[1]) : mkport(T_OP, lab, m[1]));
+    rb = var_port(m[0]);
+    rc = one ? var_port(m[0]) : var_port(m[0] + 8);
+  } else if (one) {
     L.rw[RW_OPER]++;
-    const u32 n = pnum(port);
+    rb = rc = numport(num_binary(L, n, lab, (u32)(w1 >> 32)));
+  } else if (kind == I_OP) {
+    st2_new(P, m[0], P_NONE, P_FREE);
+    st2_new(P, m[1], numport(operate_unary(lab, n)), var_port(m[0]));
+    rb = mkport(T_OP, N_SYM, m[1]);
+    rc = var_port(m[0]);
+  } else {  // I_SWITCH
+    L.rw[RW_OPER]++;
     const u32 v = num_tag(n) == N_U24 ? num_u24(n) : 0;
-    u64 w, x;
-    alloc2(L, w, x);
-    st2_new(P, w, P_NONE, P_FREE);
+    st2_new(P, m[0], P_NONE, P_FREE);
     if (v == 0) {
-      st2_new(P, x, var_port(w), P_ERA);
-      t_set(I, b, mkport(T_CTR, 0, x));
+      st2_new(P, m[1], var_port(m[0]), P_ERA);
+      rb = mkport(T_CTR, 0, m[1]);
     } else {
-      const u64 y = alloc_node(L);
-      st2_new(P, x, numport(num_new_u24(v - 1)), var_port(w));
-      st2_new(P, y, P_ERA, mkport(T_CTR, 0, x));
-      t_set(I, b, mkport(T_CTR, 0, y));
+      st2_new(P, m[1], numport(num_new_u24(v - 1)), var_port(m[0]));
+      st2_new(P, m[2], P_ERA, mkport(T_CTR, 0, m[1]));
+      rb = mkport(T_CTR, 0, m[2]);
     }
-    L.dirty = true;
-    t_set(I, c, wire_port(w));
-  } else if (port == P_ERA) {
-    count_rare(L, SC_SWITCH_ERA, 1);
-    L.rw[RW_ERAS]++;
-    t_set(I, b, P_ERA);
-    t_set(I, c, P_ERA);
-  } else {
-    u64 v, m;
-    alloc2(L, v, m);
-    st2_new(P, v, P_NONE, P_NONE);
-    st2_new(P, m, var_port(v), var_port(v + 8));
-    L.dirty = true;
-    push_link(L, np, port, mkport(T_SWI, 0, m));
-    t_set(I, b, var_port(v));
-    t_set(I, c, var_port(v + 8));
+    rc = wire_port(m[0]);
   }
+  if (!one) t_set(I, b, rb);
+  t_set(I, c, rc);
 }
 
 // A template word spec (hvm64_engine.h) as the word it stands for.  Every
@@ -952,14 +998,14 @@ DEV void exec_num(Lane &L, Interp &I, u32 kind, u32 b, u32 c, u64 w1, u64 port, 
 // exec-mask bookkeeping of every arm.  The register read uses register 0
 // for words that name none (every definition has it: t0).
 DEV u64 tspec(const Interp &I, u64 s) {
-  const u32 t = ptag(s);
-  const u64 k = paddr(s) >> 3;
-  const bool var = t == T_VAR;
-  const u64 addr = I.tbase + (var ? k >> 1 : k) * I.tstride + (var ? (k & 1) * 8 : 0);
-  const u64 rel = (s & ~ADDR_MASK) | addr;  // a slot's port; a Var spec's label is 0, so var_port(addr)
-  const bool reg = t == T_RED && s != P_NONE && s != P_FREE;
-  const u64 rv = norm_endpoint(t_get(I, reg ? (u32)k : 0u));
-  const bool lit = t == T_REF || t == T_NUM || (t == T_RED && !reg);
+  // slot, half and register numbers are small: their arithmetic is 32-bit
+  const u32 lo = (u32)s, hi = (u32)(s >> 32), t = lo & 7, k = lo >> 3, var = t == T_VAR;
+  const u64 addr = I.tbase + ((k >> var) * (u32)I.tstride + (k & var) * 8);
+  // a slot's port; a Var spec's label is 0, so var_port(addr)
+  const u64 rel = addr | t | (u64)(hi & 0xFFFF0000u) << 32;
+  const bool reg = (t == T_RED) & (hi == 0);  // P_NONE and P_FREE have high words
+  const u64 rv = norm_endpoint(t_get(I, reg ? k : 0u));
+  const bool lit = ((t == T_REF) | (t == T_NUM) | (t == T_RED)) & !reg;
   return lit ? s : reg ? rv : rel;
 }
 
@@ -976,7 +1022,6 @@ DEV void run_template(Lane &L, Interp &I, u32 off) {
   const u32 S = (u32)(h0 & 0xFF), R = (u32)((h0 >> 16) & 0xFF);
   for (u32 j = 0; j < S; j++)
     st2_new(P, I.tbase + j * I.tstride, tspec(I, HVM_TW(2 + 2 * j)), tspec(I, HVM_TW(3 + 2 * j)));
-  if (S) L.dirty = true;
   for (u32 r = 0; r < R; r++) redux(L, tspec(I, HVM_TW(2 + 2 * S + 2 * r)), tspec(I, HVM_TW(3 + 2 * S + 2 * r)));
 #undef HVM_TW
   if (h1) {
@@ -989,62 +1034,44 @@ DEV void run_template(Lane &L, Interp &I, u32 off) {
   }
 }
 
-// One instruction (instruction.rs:110-210).  The kinds that read a trg
-// (Ctr first, the most common) are tested first and the others after: a
-// wave executes the union of its lanes' paths, and each test of a per-lane
-// kind costs every lane the exec-mask bookkeeping of its branch.
+// The instruction kinds in three groups, each run by a loop of its own
+// (interp_run): the kinds that match the argument or make registers, the
+// links, and I_TEMPLATE.
+DEV bool is_link_kind(u32 kind) { return kind == I_LINK || kind == I_LINKCONST || kind == I_LINKT; }
+
+// One Ctr / Op / OpNum / Switch / Const / Wires instruction
+// (instruction.rs:110-210).  Every lane goes through the same sequence (read
+// the trg, follow it, take the node, take fresh nodes, write two registers),
+// with a branch only around what touches memory: a wave executes the union
+// of its lanes' paths.
 DEV void exec_step(Lane &L, Interp &I, u64 w0, u64 w1, u32 &np) {
   const Params &P = *L.P;
   const u32 kind = (u32)(w0 & 0xFF);
   const u32 a = (u32)(w0 >> 16) & 0xFFFF, b = (u32)(w0 >> 32) & 0xFFFF, c = (u32)(w0 >> 48);
-  const u64 t_a = t_get(I, a);  // every kind's `a` is a register of the definition (checked at book load)
-  if (kind - I_CTR <= I_SWITCH - I_CTR) {
-    // Ctr / Op / OpNum / Switch: the trg, followed if it is a wire
-    const u64 ta = (w0 & I_ASWIRE) ? as_wire(t_a) : t_a;
-    const u64 port = ptag(ta) == T_RED ? resolve(L, ta) : ta;
-    if (kind != I_CTR) {
-      exec_num(L, I, kind, b, c, w1, port, np);
-      return;
+  const bool ctr = kind == I_CTR;
+  u64 p = t_get(I, a);  // every kind's `a` is a register of the definition (checked at book load)
+  // the trg, followed if it is a wire
+  const u32 pt = ptag(p);
+  p = follow(L, p, (kind - I_CTR <= I_SWITCH - I_CTR) & ((pt == T_RED) | ((pt == T_VAR) & ((w0 & I_ASWIRE) != 0))));
+  const u32 lab = (u32)(w1 & 0xFFFF);
+  const bool match = ctr & (ptag(p) == T_CTR) & (plab(p) == lab);  // do_ctr's fast path (instruction.rs:116-121)
+  u64 x = 0, y = 0;
+  if (match) take(L, p, x, y);
+  L.rw[RW_ANNI] += match;
+  const u32 need = match ? 0 : ctr ? 2 : other_need(kind, p);
+  u64 m[3] = {0, 0, 0};
+  if (need) alloc_nodes(L, need, m);
+  if (ctr) {
+    if (!match) {  // instruction.rs:126-131
+      st2_new(P, m[0], P_NONE, P_NONE);
+      st2_new(P, m[1], var_port(m[0]), var_port(m[0] + 8));
+      push_link(L, np, p, mkport(T_CTR, lab, m[1]));
     }
-    const u32 lab = (u32)(w1 & 0xFFFF);
-    if (ptag(port) == T_CTR && plab(port) == lab) {  // do_ctr's fast path (instruction.rs:116-121)
-      u64 x, y;
-      take(L, port, x, y);
-      L.rw[RW_ANNI]++;
-      t_set(I, b, as_wire(x));
-      t_set(I, c, as_wire(y));
-      return;
-    }
-    u64 v, n;  // instruction.rs:126-131
-    alloc2(L, v, n);
-    st2_new(P, v, P_NONE, P_NONE);
-    st2_new(P, n, var_port(v), var_port(v + 8));
-    L.dirty = true;
-    push_link(L, np, port, mkport(T_CTR, lab, n));
-    t_set(I, b, var_port(v));
-    t_set(I, c, var_port(v + 8));
-    return;
+    t_set(I, b, match ? as_wire(x) : var_port(m[0]));
+    t_set(I, c, match ? as_wire(y) : var_port(m[0] + 8));
+  } else {
+    exec_other(L, I, w0, w1, p, m, np);
   }
-  if (kind == I_LINK || kind == I_LINKCONST || kind == I_LINKT) {
-    push_link(L, np, t_a, kind == I_LINK ? t_get(I, b) : kind == I_LINKT ? tspec(I, w1) : w1);
-    return;
-  }
-  if (kind == I_TEMPLATE) {
-    run_template(L, I, (u32)w1);
-    return;
-  }
-  if (kind == I_CONST) {
-    t_set(I, a, w1);
-    return;
-  }
-  // I_WIRES
-  const u64 v = alloc_node(L);
-  st2_new(P, v, P_NONE, P_NONE);
-  L.dirty = true;
-  t_set(I, a, var_port(v));
-  t_set(I, b, wire_port(v));
-  t_set(I, c, var_port(v + 8));
-  t_set(I, (u32)(w1 & 0xFFFF), wire_port(v + 8));
 }
 
 // def.rs:217-289: start the definition whose record is `d`, with t0 = `t0`.
@@ -1065,9 +1092,9 @@ DEV void interp_begin(Lane &L, Interp &I, const DefRec &d, u64 t0, u64 cdef) {
   I.Tl = HVM_TO_LDS(L.T_lds);
   I.Tg = L.T_glb;
   I.t_lds = L.lds_all || (P.t_lds && L.T_lds);
+  I.tstride = L.arenas ? 16 : TSLOT_STRIDE;
   u32 ioff = d.ioff, ilen = d.ilen, nslots = d.nslots;
   I.tbase = 0;
-  I.tstride = TSLOT_STRIDE;
   if (cdef) {
     const u32 ts = cdef_tslots(cdef);
     bool fits = false;
@@ -1076,11 +1103,10 @@ DEV void interp_begin(Lane &L, Interp &I, const DefRec &d, u64 t0, u64 cdef) {
       fits = L.a_pos + ts <= L.a_end;
       if (fits) {
         I.tbase = HVM_HEAP_OFF + L.a_pos * 16;
-        I.tstride = 16;
         L.a_pos += ts;
       }
-    } else if (L.apos + ts <= P.wave_nodes / 64) {
-      I.tbase = HVM_HEAP_OFF + (L.sub_node0 + L.apos * 64) * 16;
+    } else if (L.apos + ts <= L.slice_n) {
+      I.tbase = L.slice + (u64)L.apos * SLICE_STRIDE;
       L.apos += ts;
       fits = true;
     }
@@ -1100,25 +1126,60 @@ DEV void interp_begin(Lane &L, Interp &I, const DefRec &d, u64 t0, u64 cdef) {
   t_set(I, 0, t0);
 }
 
-// Runs instructions until the definition ends or the link list is full
-// (every instruction appends at most one link), one per loop pass:
-// fetching two per pass and stepping through them in an inner loop cost
-// register copies at the inner loop's edges (bitonic 2^16 -2%).
+// The next instruction's two words.
+DEV void fetch(const Lane &L, const Interp &I, u64 &w0, u64 &w1) {
+  if (has_book(L)) {
+    w0 = L.book[L.book_ins + I.ipw];
+    w1 = L.book[L.book_ins + I.ipw + 1];
+  } else {
+    w0 = L.P->instrs[I.ipw];
+    w1 = L.P->instrs[I.ipw + 1];
+    HVM_SETTLE_LOADS();
+  }
+}
+
+// Runs instructions until the definition ends or the link list is full.
+// A wave executes the union of what its lanes do at one step, so the kinds
+// run in three loops, each reconverging before the next: every lane's
+// pattern steps; then the templates of all the lanes that reached theirs, at
+// once; then the links.  A compiled program has exactly that order, so its
+// lanes go through once; an interpreted program, whose links stand among its
+// patterns, goes round again.
 DEV void interp_run(Lane &L, Interp &I, u32 &np) {
   HVM_SETTLE_LOADS();
+  u64 w0 = 0, w1 = 0;
   while (I.left > 0 && np < LINK_CAP) {
-    u64 w0, w1;
-    if (has_book(L)) {
-      w0 = L.book[L.book_ins + I.ipw];
-      w1 = L.book[L.book_ins + I.ipw + 1];
-    } else {
-      w0 = L.P->instrs[I.ipw];
-      w1 = L.P->instrs[I.ipw + 1];
-      HVM_SETTLE_LOADS();
-    }
+    fetch(L, I, w0, w1);
+    const u32 kind = (u32)(w0 & 0xFF);
+    if (kind == I_TEMPLATE || is_link_kind(kind)) break;
     exec_step(L, I, w0, w1, np);
     I.ipw += 2;
     I.left -= 1;
+  }
+  if (I.left > 0 && np < LINK_CAP && (u32)(w0 & 0xFF) == I_TEMPLATE) {
+    run_template(L, I, (u32)w1);
+    I.ipw += 2;
+    I.left -= 1;
+  }
+  while (I.left > 0 && np < LINK_CAP) {
+    fetch(L, I, w0, w1);
+    const u32 kind = (u32)(w0 & 0xFF);
+    if (!is_link_kind(kind)) break;
+    const u64 t_a = t_get(I, (u32)(w0 >> 16) & 0xFFFF);
+    push_link(L, np, t_a,
+              kind == I_LINK ? t_get(I, (u32)(w0 >> 32) & 0xFFFF) : kind == I_LINKT ? tspec(I, w1) : w1);
+    I.ipw += 2;
+    I.left -= 1;
+  }
+}
+
+// The running definition (if any) to its end, and every link the task asks
+// for.
+DEV void run_program(Lane &L, Interp &I, u32 &np) {
+  for (;;) {
+    if (I.left > 0) interp_run(L, I, np);
+    if (np == LINK_CAP || I.left == 0) flush_links(L, np);
+    if (I.left == 0) break;
   }
 }
 
@@ -1130,9 +1191,9 @@ DEV void expand_call(Lane &L, Interp &I, u32 &np, u64 cell, u64 port) {
   if (ptag(port) == T_REF && port != P_ERA) {
     u64 oaddr = paddr(port);
     if (addr_in_heap(oaddr)) {
-      u64 x = ld(P, cell), y = ld(P, oaddr);
-      st(P, cell, P_FREE);
-      st(P, oaddr, P_FREE);
+      u64 x = ld(L, cell), y = ld(L, oaddr);
+      st(L, cell, P_FREE);
+      st(L, oaddr, P_FREE);
       push_link(L, np, x, y);
       return;
     }
@@ -1146,23 +1207,22 @@ DEV void expand_call(Lane &L, Interp &I, u32 &np, u64 cell, u64 port) {
     interp_begin(L, I, load_def(L, def_index(oaddr)), expand_ref(cell), load_cdef(L, def_index(oaddr)));
     return;
   }
-  u64 out = ld(P, cell);
-  st(P, cell, P_FREE);
+  u64 out = ld(L, cell);
+  st(L, cell, P_FREE);
   u32 t = ptag(port);
   if (t == T_REF || t == T_NUM || t == T_VAR || t == T_RED) {
     push_link(L, np, out, port);
     return;
   }
-  u64 p1, p2;
+  u64 p1, p2, m[3];
   take(L, port, p1, p2);
-  u64 v1 = alloc_vars2(L), e1 = alloc_node(L);
-  u64 v2 = v1 + 8, e2 = e1 + 8;
-  st2(P, e1, var_port(v1), var_port(v2));
-  L.dirty = true;
-  u64 n = new_node(L, t, plab(port), var_port(v1), var_port(v2));
-  push_link(L, np, out, n);
-  push_link(L, np, p1, expand_ref(e1));
-  push_link(L, np, p2, expand_ref(e2));
+  alloc_nodes(L, 3, m);  // the node's var cells, the two ExpandDefs' cells, the node
+  st2_new(P, m[0], P_NONE, P_NONE);
+  st2_new(P, m[1], var_port(m[0]), var_port(m[0] + 8));
+  st2_new(P, m[2], var_port(m[0]), var_port(m[0] + 8));
+  push_link(L, np, out, mkport(t, plab(port), m[2]));
+  push_link(L, np, p1, expand_ref(m[1]));
+  push_link(L, np, p2, expand_ref(m[1] + 8));
 }
 
 // def.rs:177-189
@@ -1179,95 +1239,51 @@ DEV void capture_redex(Lane &L, u64 port, u64 trg) {
   HVM_ST(&P.captured[2 * i + 1], trg);
 }
 
-DEV void call(Lane &L, Interp &I, u32 &np, u64 port, u64 trg) {
+// The redexes of the call rings: a Ref that is not the eraser on at least
+// one side.  The arms of interact.rs:6-44 that apply, in their order: of two
+// nilary ports the first one that is not skippable is called (neither: an
+// erasure); of a nilary port and a node, the Ref is called, unless the node
+// is a Ctr whose label is not below the Ref's (comm02).  Then Net::call
+// (def.rs:177-189): a Ctr whose label the definition's set does not hold is
+// copied too; anything else starts the definition.
+DEV void call_redex(Lane &L, Interp &I, u32 &np, u64 a, u64 b) {
   const Params &P = *L.P;
-  u64 addr = paddr(port);
-  if (addr_in_heap(addr)) {  // ExpandDef: LabSet::ALL
-    if (ptag(trg) == T_CTR && plab(trg) >= 0xFFFF) {
-      comm02(L, np, port, trg);
-      return;
-    }
-    L.rw[RW_DREF]++;
-    expand_call(L, I, np, addr, trg);
+  const u32 at = ptag(a), bt = ptag(b);
+  const bool aref = (at == T_REF) & (a != P_ERA);
+  const bool nil = !is_binary(a) & !is_binary(b);
+  const bool call_a = nil ? aref & !is_skippable(a) : aref;
+  const u64 port = call_a ? a : b, trg = call_a ? b : a;
+  if (nil & is_skippable(port)) {
+    L.rw[RW_ERAS]++;
     return;
   }
-  u32 di = def_index(addr);
-  if (addr == 0 || di >= P.ndefs) {
-    fail(L, ERR_BADPTR, BAD_DEF_CALL);
-    return;
-  }
-  const DefRec d = load_def(L, di);
-  if (ptag(trg) == T_CTR && !labs_has(L, d, plab(trg))) {
+  const u64 addr = paddr(port);
+  const bool ctr = ptag(trg) == T_CTR;
+  const u32 lab = plab(trg);
+  const u32 di = def_index((u64)(u32)addr);
+  const bool heap = addr_in_heap(addr), def = !heap & (addr != 0) & (di < P.ndefs);
+  const DefRec d = load_def(L, def ? di : 0);
+  const u64 cdef = load_cdef(L, def ? di : 0);
+  const bool copy = ctr & ((lab >= plab(port)) | (def && !labs_has(L, d, lab)));
+  if (copy) {
     comm02(L, np, port, trg);
     return;
   }
+  if (!def && !heap) {
+    fail(L, ERR_BADPTR, BAD_DEF_CALL);
+    return;
+  }
   L.rw[RW_DREF]++;
+  if (heap) {  // ExpandDef: LabSet::ALL
+    expand_call(L, I, np, addr, trg);
+    return;
+  }
   if (d.flags & DEF_INERT) {  // InertDef::call (pre_reduce.rs:108-115)
     capture_redex(L, port, trg);
     return;
   }
-  interp_begin(L, I, d, trg, load_cdef(L, di));
+  interp_begin(L, I, d, trg, cdef);
 }
-
-// interact.rs:6-44.  The arms are tested in the reference's order; each arm
-// picks a rule and which side goes first, and every rule has a single call
-// site (code size: the rules are inlined once).
-enum Rule : u32 { R_UNIMPL, R_CALL, R_ERAS, R_COMM22, R_ANNI, R_COMM02, R_OPNUM, R_SWITCHNUM };
-
-DEV u32 choose_rule(u64 a, u64 b, bool &swap) {
-  u32 at = ptag(a), bt = ptag(b);
-  bool anil = at == T_REF || at == T_NUM, bnil = bt == T_REF || bt == T_NUM;
-  swap = false;
-  if (at <= T_VAR || bt <= T_VAR) return R_UNIMPL;
-  if (at == T_REF && bnil && !is_skippable(a)) return R_CALL;
-  if (anil && bt == T_REF && !is_skippable(b)) { swap = true; return R_CALL; }
-  if (anil && bnil) return R_ERAS;
-  if (at == T_CTR && bt == T_SWI && plab(a) != 0) return R_COMM22;
-  if (at == T_SWI && bt == T_CTR && plab(b) != 0) return R_COMM22;
-  if ((at == T_CTR && bt == T_OP) || (at == T_OP && bt == T_CTR)) return R_COMM22;
-  if (at == T_CTR && bt == T_CTR && plab(a) != plab(b)) return R_COMM22;
-  if (at == bt && (at == T_SWI || at == T_OP || at == T_CTR)) return R_ANNI;
-  if (at == T_REF && bt == T_CTR && plab(b) >= plab(a)) return R_COMM02;
-  if (at == T_CTR && bt == T_REF && plab(a) >= plab(b)) { swap = true; return R_COMM02; }
-  if (at == T_NUM && bt == T_CTR) return R_COMM02;
-  if (at == T_CTR && bt == T_NUM) { swap = true; return R_COMM02; }
-  if (a == P_ERA) return R_COMM02;
-  if (b == P_ERA) { swap = true; return R_COMM02; }
-  if (at == T_REF) return R_CALL;
-  if (bt == T_REF) { swap = true; return R_CALL; }
-  if (at == T_OP && bt == T_NUM) return R_OPNUM;
-  if (at == T_NUM && bt == T_OP) { swap = true; return R_OPNUM; }
-  if (at == T_SWI && bt == T_NUM) return R_SWITCHNUM;
-  if (at == T_NUM && bt == T_SWI) { swap = true; return R_SWITCHNUM; }
-  return R_UNIMPL;  // Switch-Ctr(0), Op-Switch: unimplemented!() in the reference
-}
-
-DEV void interact(Lane &L, Interp &I, u32 &np, u64 a, u64 b) {
-  bool swap;
-  const u32 rule = choose_rule(a, b, swap);
-  if (swap) {
-    u64 t = a;
-    a = b;
-    b = t;
-  }
-  switch (rule) {
-    case R_CALL: call(L, I, np, a, b); break;
-    case R_ERAS: L.rw[RW_ERAS]++; break;
-    case R_COMM22: comm22(L, np, a, b); break;
-    case R_ANNI: anni2(L, np, a, b); break;
-    case R_COMM02: comm02(L, np, a, b); break;
-    case R_OPNUM: op_num(L, np, a, b); break;
-    case R_SWITCHNUM: switch_num(L, np, a, b); break;
-    default: fail(L, ERR_UNIMPL); break;
-  }
-}
-
-// One lane's whole task: interact the redex (a, b) when `has`, else run
-// definition `di` with t0 (when di != NO_DEF), then link everything the task
-// asks for.  The loop alternates instructions and link rounds until the
-// definition (if any) has ended and the link list is empty; the link code is
-// shared by every rule and instruction.
-static const u32 NO_DEF = 0xFFFFFFFFu;
 
 // Serving: slot `s`'s net is normal.  Its root port (following parked
 // ports) and tag go to the completion ring in host memory (the entry's
@@ -1276,7 +1292,7 @@ DEV void serve_complete(Lane &L, u32 s) {
   const Params &P = *L.P;
   u64 p = var_port(HVM_LD(&P.slot_root[s]));
   for (u32 hop = 0; hop < MAX_CHAIN && is_endpoint(p); hop++) {
-    const u64 v = ld(P, paddr(p));
+    const u64 v = ld(L, paddr(p));
     if (v == P_NONE) break;
     p = v;
   }
@@ -1323,82 +1339,106 @@ DEV void serve_settle(Lane &L) {
   L.acct_delta = 0;
 }
 
-DEV void serve_account(Lane &L, u32 delta) {
-  if (delta == 0) return;
-  // always waited for, increments too: an increment still in flight when a
-  // lane of another iteration consumes the redex could let the count reach
-  // 0 early (measured: early completions, then a reused slot's stale redexes)
-  const u32 old = HVM_FAA(&L.P->pending[L.cur_net], delta);
-  if (old + delta == 0) serve_complete(L, L.cur_net);
-}
+static const u32 NO_DEF = 0xFFFFFFFFu;
 
-// The instructions and link rounds of a task, then (serving) the redexes
-// without a heap port it made, each interacted here in turn.
-DEV void task_loop(Lane &L, Interp &I, u32 &np) {
-  for (;;) {
-    for (;;) {
-      if (I.left > 0) interp_run(L, I, np);
-      if (np > 0) flush_links(L, np);
-      if (I.left == 0) break;
-    }
-    if (!L.serve || L.inl_n == 0) break;
-    L.inl_n--;
-    interact(L, I, np, L.inl[2 * L.inl_n], L.inl[2 * L.inl_n + 1]);
-  }
-}
-
-DEV void run_task(Lane &L, bool has, u64 a, u64 b, u32 di, u64 t0) {
+DEV Interp interp_none(const Lane &L) {
   Interp I;
   I.left = 0;
   I.ipw = 0;
   I.Tl = nullptr;
   I.Tg = nullptr;
   I.t_lds = L.lds_all;  // a constant where the kernel knows it
-  u32 np = 0;
-  if (has && L.arenas) L.cur_net = net_of_port(*L.P, a, net_of_port(*L.P, b, L.cur_net));
-  if (L.serve) {
-    L.pushed = 0;
-    L.a_net = NO_NET;  // a slot's arena restarts when its net completes
-  }
-  if (has) interact(L, I, np, a, b);
-  else if (di != NO_DEF) interp_begin(L, I, load_def(L, di), t0, load_cdef(L, di));
-  task_loop(L, I, np);
-  // nodes a template wrote may be reached only through the redexes it
-  // pushed: retire their stores before any lane reads them
-  publish_if_dirty(L);
-  if (L.serve && has) serve_account_deferred(L, L.pushed - 1u);
+  I.tbase = 0;
+  I.tstride = L.arenas ? 16 : TSLOT_STRIDE;
+  return I;
 }
 
-// Serving: boots request `tag` (definition di) into free slot s, as
-// Net::boot + the expansion of Net::normal (net.rs:30-32, 55-69) would.  The
-// slot's count is held at 1 while the boot runs, so that a redex the boot
-// sends to the global ring cannot complete the net early.
-DEV void serve_boot(Lane &L, u32 s, u32 di, u64 tag) {
+// Runs definition `di` with t0 (Net::boot, Host::encode_net), outside the
+// reduction kernel.
+DEV void run_def(Lane &L, u32 di, u64 t0) {
+  Interp I = interp_none(L);
+  u32 np = 0;
+  interp_begin(L, I, load_def(L, di), t0, load_cdef(L, di));
+  run_program(L, I, np);
+  // nodes a template wrote may be reached only through the redexes it
+  // pushed: retire their stores before any lane reads them
+  publish();
+}
+
+// What bounds an iteration is the instructions one wave issues (a few
+// thousand, four cycles each) plus its dependent round trips to memory
+// (about 1,000 cycles each); the lane's state is therefore small, its rare
+// parts are in LDS, and nothing on the way is a function call: every call
+// and every divergent merge costs moves of whatever lives across it.  With
+// the state in registers, calls in the access path and one interaction
+// switch for all classes, an iteration of rules that read one node took
+// 9,240 cycles and a call iteration 27,800; this way 7,000 and 26,200
+// (bitonic 2^6: 8.32 -> 7.08 ms, 2^16: 118 -> 109 ms, tree-sum 18: 5.46 ->
+// 4.70 ms).
+//
+// One iteration of a wave: every lane with `has` runs the redex (a, b) of
+// ring class `cls` (wave-uniform: each class has its code, entered by a
+// scalar branch), then links everything it asks for.  Serving: then the
+// redexes without a heap port that made, each in turn (they are calls: a
+// pair of which neither side can be called was dropped).  `booting`
+// (serving): the lane starts definition `di` with `t0` instead, its net's
+// root link already in the list.
+DEV void run_tasks(Lane &L, u32 cls, bool has, u64 a, u64 b, bool booting, u32 di, u64 t0, u32 np) {
+  Interp I = interp_none(L);
+  if (L.arenas && has) L.cur_net = net_of_port(*L.P, a, net_of_port(*L.P, b, L.cur_net));
+  if (L.serve) {
+    L.pushed = 0;
+    if (!booting) L.a_net = NO_NET;  // a slot's arena restarts when its net completes
+  }
+  for (;;) {
+    if (cls == CLS_ANNI) {
+      if (has) anni2(L, np, a, b);
+      flush_links(L, np);
+    } else if (cls == CLS_COMM) {
+      if (has) comm22(L, np, a, b);
+      flush_links(L, np);
+    } else if (cls == CLS_OTHER) {
+      if (has) rule_other(L, np, a, b);
+      flush_links(L, np);
+    } else {
+      if (has) call_redex(L, I, np, a, b);
+      if (L.serve && booting) interp_begin(L, I, load_def(L, di), t0, load_cdef(L, di));
+      run_program(L, I, np);
+    }
+    if (!L.serve) break;
+    has = L.inl_n > 0;
+    if (!HVM_ANY(has)) break;
+    if (has) {
+      L.inl_n--;
+      a = L.inl[2 * L.inl_n];
+      b = L.inl[2 * L.inl_n + 1];
+    }
+    cls = CLS_CALL;
+    booting = false;
+  }
+  publish();
+}
+
+// Serving: sets a lane up to boot a request into free slot s as Net::boot +
+// the expansion of Net::normal (net.rs:30-32, 55-69) would; run_tasks then
+// runs its definition with the port returned as t0, the link of the new root
+// already in the list.  The slot's count is held at 1 while the boot runs,
+// so that a redex the boot sends to the global ring cannot complete the net
+// early.
+DEV u64 serve_boot(Lane &L, u32 s, u64 tag, u32 &np) {
   const Params &P = *L.P;
   L.cur_net = s;
   L.a_net = NO_NET;
   HVM_FAA(&P.pending[s], 1u);
   HVM_ST(&P.slot_tag[s], tag);
-  const u64 r2 = alloc_node(L);
-  st2(P, r2, P_NONE, var_port(r2));
-  HVM_ST(&P.slot_root[s], r2);
-  const u64 r = alloc_var1(L);
+  u64 m[2];
+  alloc_nodes(L, 2, m);
+  st2_new(P, m[0], P_NONE, var_port(m[0]));
+  st2_new(P, m[1], P_NONE, P_FREE);
+  HVM_ST(&P.slot_root[s], m[0]);
   L.rw[RW_DREF]++;
-  Interp I;
-  I.left = 0;
-  I.ipw = 0;
-  I.Tl = nullptr;
-  I.Tg = nullptr;
-  I.t_lds = L.lds_all;  // a constant where the kernel knows it
-  u32 np = 0;
-  L.pushed = 0;
-  interp_begin(L, I, load_def(L, di), var_port(r), load_cdef(L, di));
-  task_loop(L, I, np);
-  push_link(L, np, var_port(r), expand_ref(r2 + 8));
-  task_loop(L, I, np);
-  publish_if_dirty(L);
-  publish();
-  serve_account(L, L.pushed - 1u);
+  push_link(L, np, var_port(m[1]), expand_ref(m[0] + 8));
+  return var_port(m[1]);
 }
 
 // ---------------------------------------------------------------------------
@@ -1406,15 +1446,16 @@ DEV void serve_boot(Lane &L, u32 s, u32 di, u64 tag) {
 // ---------------------------------------------------------------------------
 DEV void lane_init(Lane &L, const Params &P, u32 gwave, u32 lane) {
   L.P = &P;
-  L.sub_node0 = P.ring_node0 + (u64)gwave * P.wave_nodes + lane;
+  L.slice = HVM_HEAP_OFF + (P.ring_node0 + (u64)gwave * P.wave_nodes + lane) * 16;
+  L.slice_n = (u32)(P.wave_nodes / 64);
   L.apos_home = &P.alloc_pos[(u64)gwave * 64 + lane];
-  L.apos = *L.apos_home;
+  L.apos = (u32)*L.apos_home;
   L.slice_rest = 0;
   L.ov_left = 0;
   L.ov_cur = 0;
   L.fcn = 0;
-  L.fc0 = L.fc1 = L.fc2 = L.fc3 = 0;
-  L.dirty = false;
+  L.FC = nullptr;
+  L.in_lds = false;
   L.arenas = P.gmap != nullptr;
   L.cur_net = 0;
   L.serve = false;  // set by the serving kernel
@@ -1441,8 +1482,13 @@ DEV void lane_init(Lane &L, const Params &P, u32 gwave, u32 lane) {
   L.book_tmpl = 0;
 #pragma unroll
   for (u32 k = 0; k < RW_SLOTS; k++) L.rw[k] = 0;
+  L.bad = 0;
+  L.err = 0;
 }
 
-DEV void lane_finish(Lane &L) { *L.apos_home = L.apos; }
+DEV void lane_finish(Lane &L) {
+  *L.apos_home = L.apos;
+  lane_report(L);
+}
 
 }  // namespace hvm

@@ -109,7 +109,7 @@ enum : u32 {
 
 // Global control block.  Hot words sit on separate 128-byte lines.
 struct alignas(128) Globals {
-  u64 S;           // (queued redexes << 32) | active waves
+  u64 S;           // (queued redexes << 32) | blocks with an active wave
   u64 _p0[15];
   u64 q_head;      // next slot to consume in the global redex ring
   u64 _p1[15];
@@ -224,7 +224,8 @@ static const u32 SERVE_INL = 32;
 static const u32 SERVE_SUB = 8;
 
 // Mailbox of a wave: a count word on its own 128-byte line, then up to
-// MBOX_PAIRS redex pairs handed to the wave by another wave.
+// MBOX_PAIRS redex pairs handed to the wave by another wave (a zero word: not
+// there yet; the receiver zeroes what it has read).
 static const u32 MBOX_PAIRS = 64;
 static const u32 MBOX_WORDS = 16 + 2 * MBOX_PAIRS;
 // Count word value written to every mailbox by the wave that ends the

@@ -181,8 +181,24 @@ __global__ void k_expand(Params P, u64 old_root_cell) {
 // with more than one iteration's worth of redexes spills the excess (the
 // oldest redexes of its fullest class) to the global ring while other waves
 // are idle; an empty wave claims up to 64 redexes from the global ring.
-// S = (queued << 32) | active waves; the reduction is complete when S == 0,
-// a state no wave can leave.  S is one word shared by every wave and its
+//
+// Sharing.  A pass runs one ring, so a wave with several takes as many passes
+// for what is ready at once.  While waves of its block are idle it hands each
+// a whole ring, through LDS (s_idle, s_given: no memory traffic, seen within
+// 0.1 us); while few blocks are active (SHARE_BLOCKS), another ring goes to an
+// idle wave elsewhere, through its mailbox.  With more blocks active the
+// atomics on S and the idle set cost more than the passes they save (bitonic
+// 2^16: 113 ms; sharing beyond the block without that bound 220 ms), and a
+// batch whose global ring is stocked does not share at all: there fuller
+// passes count.  Measured without and with: Church c2^c9 4.50 -> 3.45 ms,
+// bitonic 2^6 7.08 -> 5.67 ms, 2^11 32.2 -> 28.4 ms, tree-sum 10 1.02 -> 0.84
+// ms; 2^16 109 -> 112 ms (shorter but more passes).
+//
+// S = (queued << 32) | active blocks; the reduction is complete when S == 0,
+// a state no wave can leave.  A block is active while one of its waves is:
+// s_act counts those, the wave that makes it 0 takes the block's count off S,
+// and a wave that claims from the global ring or is sent mail brings a count
+// with it, which goes back if the block has one.  S is one word shared by every wave and its
 // device-scope accesses all go to one memory channel, so busy waves touch it
 // only to spill (and read it every 64 iterations).  Idle waves poll their own
 // mailbox and read S only every IDLE_CHECK polls (for redexes on the global
@@ -194,16 +210,20 @@ __global__ void k_expand(Params P, u64 old_root_cell) {
 // mailboxes are off and idle waves poll S with a growing, jittered backoff
 // capped near 1 ms.
 static const u32 REFRESH = 64;        // busy iterations between control-word reads
-static const u32 MAX_BACKOFF = 16384;  // idle backoff cap, in s_sleep(2) units (~0.9 ms)
-static const u32 MBOX_POLL = 16;       // s_sleep(2) units between mailbox polls (~1 us)
+static const u32 MAX_BACKOFF = 8192;   // idle backoff cap, in looks at the block's LDS words (~0.9 ms)
+static const u32 MBOX_POLL = 8;        // looks at the block's LDS words between mailbox polls (~1 us)
+static const u32 SHARE_BLOCKS = 64;     // active blocks up to which rings are shared beyond the block
 static const u32 IDLE_CHECK = 1024;    // mailbox polls between reads of S (a power of two)
 // Defaults of the tunable thresholds (Params::mbox_keep, Params::fill_below).
 static const u32 MBOX_KEEP = 256;      // redexes a busy wave keeps before handing some off
 static const u32 FILL_BELOW = 32;      // batched nets: pending redexes under which a busy wave claims
 
-DEV void wave_sleep(u32 units) {
-  for (u32 z = 0; z < units; z++) __builtin_amdgcn_s_sleep(2);
-}
+// Words in LDS that the block's waves share.
+DEV u32 lds_get(const u32 *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+DEV void lds_put(u32 *p, u32 v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+DEV u32 lds_add(u32 *p, u32 v) { return __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+DEV u32 lds_and(u32 *p, u32 v) { return __hip_atomic_fetch_and(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
+DEV void lds_or(u32 *p, u32 v) { (void)__hip_atomic_fetch_or(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 
 // Wave-wide values for the scheduler.  A loop pass reads about twenty of
 // them; through LDS (ds_bpermute, what __shfl compiles to) each costs its
@@ -263,6 +283,32 @@ DEV void claim_global(const Params &P, Lane &L, pair *bag, u32 *top_c, u32 k, u3
     const u32 idx = HVM_LDS_FAA(&top_c[c], 1u);
     bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
   }
+}
+
+// Takes the k (<= 64) redexes delivered to the wave's mailbox into its rings
+// (which hold at most 64, so every ring has room).
+DEV void take_mail(u64 *box, Lane &L, pair *bag, u32 *top_c, u32 k, u32 lane, u64 t_end) {
+  if (lane < k) {
+    u64 *const e = box + 16 + 2 * lane;
+    u64 a, b;
+    for (;;) {  // the sender's stores of the pairs are on their way
+      a = gld(e);
+      b = gld(e + 1);
+      if (a != 0 && b != 0) break;
+      if (wall_clock64() > t_end) {
+        fail(L, ERR_TIMEOUT);
+        a = b = P_ERA;  // skippable pair: dropped without effect
+        break;
+      }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    st16(e, 0, 0);  // (retired before this wave can be sent mail again: it runs a task first)
+    const u32 c = redex_class(a, b, L.book, has_book(L), L.P->ndefs);
+    const u32 idx = HVM_LDS_FAA(&top_c[c], 1u);
+    bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
+  }
+  if (lane == 0) gst(box, 0);
+  __builtin_amdgcn_wave_barrier();
 }
 
 DEV u64 spill_to_global(const Params &P, const pair *bag, u32 *bot_c, u32 c, u32 cnt, u32 lane, u32 bot, u32 &err) {
@@ -355,6 +401,15 @@ DEV bool serve_waiting(const Params &P, u32 lane) {
   return uniform(w) != 0;
 }
 
+// A wave runs the ring with the largest key: the fullest of the anni / comm /
+// other rings if any holds redexes (they are cheap and release the work
+// behind them, and definition calls meanwhile gather into fuller
+// iterations), else the fullest definition-call ring; lowest index on ties.
+// (n << 4 | 15 - index in the low 24 bits.)
+DEV u32 ring_key(u32 c, u32 n) {
+  return ((c < CLS_CALL && n > 0) ? 1u << 24 : 0u) | (n << 4) | (15 - c);
+}
+
 // ARENAS: compiled for per-net arenas (P.gmap set) or for the per-lane
 // allocation rings; each instantiation carries only its mode's allocator.
 // SERVE: the serving launch (arenas are request slots; the kernel runs until
@@ -373,6 +428,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   __shared__ u32 s_top[WAVES_PER_BLOCK][NCLS];
   __shared__ u32 s_bot[WAVES_PER_BLOCK][NCLS];
   __shared__ u64 s_book[BOOK_LDS_WORDS];
+  // sharing inside the block: its active waves; the waves a redex ring may be
+  // handed to (bit per wave); per wave, that one was
+  __shared__ u32 s_act, s_idle, s_given[WAVES_PER_BLOCK];
   const u32 wib = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // the book, copied into LDS when it fits (the host decides: P.book_lds)
   const u32 nd = P.ndefs * 4;
@@ -385,17 +443,21 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     for (u32 i = threadIdx.x; i < P.ndefs; i += blockDim.x) s_book[b_cdef + i] = P.cdefs[i];
     for (u32 i = threadIdx.x; i < P.tmpl_words; i += blockDim.x) s_book[b_tmpl + i] = P.tmpl[i];
   }
+  if (threadIdx.x == 0) {
+    s_act = 0;
+    s_idle = (1u << WAVES_PER_BLOCK) - 1;
+  }
+  if (threadIdx.x < WAVES_PER_BLOCK) s_given[threadIdx.x] = 0;
+  if (threadIdx.x < WAVES_PER_BLOCK * NCLS) {
+    s_top[threadIdx.x / NCLS][threadIdx.x % NCLS] = 0;
+    s_bot[threadIdx.x / NCLS][threadIdx.x % NCLS] = 0;
+  }
   __syncthreads();
   const u32 gwave = blockIdx.x * WAVES_PER_BLOCK + wib;
   Globals *g = P.g;
   pair *bag = s_bag[wib];
   u32 *top_c = s_top[wib];
   u32 *bot_c = s_bot[wib];
-  if (lane < NCLS) {
-    top_c[lane] = 0;
-    bot_c[lane] = 0;
-  }
-  __builtin_amdgcn_wave_barrier();
   Lane L;
   lane_init(L, P, gwave, lane);
   L.arenas = ARENAS;
@@ -428,18 +490,49 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   // fills at the same pace (with lane i taking the i-th redex, low lanes ran
   // nearly every task and lapped their slices long before the others).
   u32 rot = 0;
-  u64 S_cache = 0;             // last value of S seen by this wave
+  // last value of S seen by this wave (a batch's ring is taken to be stocked
+  // until it has looked)
+  u64 S_cache = P.fill ? 1ull << 32 : 0;
   u64 S_next = 0;              // lane 0: control words read at iteration end
   u32 err_next = 0;
   bool fresh = false;          // S_next / err_next hold a read to consume
+  // lane i < idle_words: word i of the idle set as last seen
+  u64 idle_word = lane < P.idle_words ? ~0ull >> (lane == P.idle_words - 1 ? (64 - (P.total_waves & 63)) & 63 : 0) : 0;
   u64 st[ST_SLOTS] = {};
   // mailboxes: off under a reduce(limit) budget (a wave that stops there
   // must not have a delivery in flight)
   const bool use_mbox = !limited && P.mbox != nullptr && P.idle_bits != nullptr;
   u64 *my_box = use_mbox ? P.mbox + (u64)gwave * MBOX_WORDS : nullptr;
   bool in_set = false;         // this wave's bit is set in P.idle_bits
+  bool mail_due = false;       // a sender took the bit: a delivery is on its way
   u32 idle_polls = 0;
+  u32 idle_ticks = 0;          // idle passes until the next look at global memory
   u32 admit_tick = 0;          // serving, wave 0: busy iterations since the last admission
+  const u32 my_bit = 1u << wib;
+  // This wave becomes active: it counts in s_act, and a count it holds in S
+  // becomes the block's, or goes back when the block has one.  (The count
+  // goes back long before the block's own can: every task retires its
+  // wave's memory operations.)
+  auto enter = [&](bool counted) {
+    u32 was = 0;
+    if (lane == 0) was = lds_add(&s_act, 1u);
+    if (counted && uniform(was) > 0 && lane == 0)
+      __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    active = true;
+  };
+  // This wave is no longer one that can be handed a ring; false: it just was
+  // handed one (a sibling that took the bit is a running wave about to
+  // deliver, so the wait is short).
+  auto leave_block_idle = [&]() {
+    u32 old = 0;
+    if (lane == 0) old = lds_and(&s_idle, ~my_bit);
+    if (uniform(old) & my_bit) return true;
+    while (uniform(lds_get(&s_given[wib])) == 0 && wall_clock64() <= t_end) __builtin_amdgcn_s_sleep(1);
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    if (lane == 0) lds_put(&s_given[wib], 0u);
+    active = true;  // the sibling counted it
+    return false;
+  };
   if (use_mbox) {  // every wave starts idle: in the idle set, not counted in S
     if (lane == 0)
       __hip_atomic_fetch_or(&P.idle_bits[gwave >> 6], 1ull << (gwave & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -473,7 +566,8 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // ring occupancy: lane c < NCLS reads class c
     u32 my_top = lane < NCLS ? top_c[lane] : 0, my_bot = lane < NCLS ? bot_c[lane] : 0;
     u32 my_n = my_top - my_bot;
-    u32 n = row0_sum(my_n);
+    // (an idle wave's rings are empty, or a sibling is just writing them)
+    u32 n = active ? row0_sum(my_n) : 0;
 
     // ---- empty rings: idle.  An idle wave is in the idle set (its bit in
     // P.idle_bits) and polls its own mailbox, where a busy wave can hand it
@@ -482,18 +576,28 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // the global ring, errors and the deadline.
     if (n == 0 && !admitting) {
       if (active) {
-        if (use_mbox && lane == 0)
-          __hip_atomic_fetch_or(&P.idle_bits[gwave >> 6], 1ull << (gwave & 63), __ATOMIC_RELAXED,
-                                __HIP_MEMORY_SCOPE_AGENT);
-        in_set = use_mbox;
-        u64 old = 0;
-        if (lane == 0) old = __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        S_cache = uniform(old) - 1;
+        if (use_mbox && !in_set && !mail_due) {
+          if (lane == 0)
+            __hip_atomic_fetch_or(&P.idle_bits[gwave >> 6], 1ull << (gwave & 63), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+          in_set = true;
+        }
+        u32 was = 0;
+        if (lane == 0) {
+          lds_or(&s_idle, my_bit);
+          was = lds_add(&s_act, ~0u);
+        }
         active = false;
         idle_polls = 0;
+        idle_ticks = 0;
+        if (uniform(was) == 1) {  // the block's last active wave
+          u64 old = 0;
+          if (lane == 0) old = __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          S_cache = uniform(old) - 1;
+        }
         // nothing active, nothing queued: done (serving: once the host has
         // asked to stop)
-        bool end = S_cache == 0;
+        bool end = uniform(was) == 1 && S_cache == 0;
         if (SERVE && end) {
           u64 stop = 0;
           if (lane == 0) stop = HVM_LD_SYS(&P.host_ctl[SH_STOP]);
@@ -507,26 +611,35 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           break;
         }
       }
+      // a ring from a wave of this block: looked for between the looks at
+      // global memory
+      bool given = uniform(lds_get(&s_given[wib])) != 0;
+      for (; !given && idle_ticks > 0; idle_ticks--) {
+        __builtin_amdgcn_s_sleep(1);
+        given = uniform(lds_get(&s_given[wib])) != 0;
+      }
+      if (given) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+        if (lane == 0) lds_put(&s_given[wib], 0u);
+        active = true;  // counted by the sibling, which also took the bit in s_idle
+        backoff = 1 + (gwave & 7);
+        continue;
+      }
       if (TIMING) st[ST_IDLE_IT]++;
       if (use_mbox) {
         u64 k = 0;
         if (lane == 0) k = gld(my_box);
         k = uniform(k);
         if (k == MBOX_DONE) break;
-        if (k > 0) {  // a delivery: the sender already counted this wave active
-          if (lane < k) {
-            const u64 a = gld(my_box + 16 + 2 * lane), b = gld(my_box + 16 + 2 * lane + 1);
-            const u32 c = redex_class(a, b, L.book, has_book(L), P.ndefs);  // the rings are empty: k <= 64 entries fit
-            const u32 idx = HVM_LDS_FAA(&top_c[c], 1u);
-            bag[ring_base(c) + (idx & (ring_cap(c) - 1))] = pair{a, b};
-          }
-          if (lane == 0) gst(my_box, 0);
+        if (k > 0) {  // a delivery: the sender took this wave out of the idle set and counted it in S
+          if (leave_block_idle()) enter(true);
+          else if (lane == 0) __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          take_mail(my_box, L, bag, top_c, (u32)k, lane, t_end);
           if (TIMING) st[ST_CLAIMS]++;
           if (TIMING) st[ST_CLAIMED] += k;
-          active = true;
           in_set = false;
+          mail_due = false;
           backoff = 1 + (gwave & 7);
-          __builtin_amdgcn_wave_barrier();
           continue;
         }
       }
@@ -543,10 +656,14 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
                                          __HIP_MEMORY_SCOPE_AGENT);
           left = ((uniform(old) >> (gwave & 63)) & 1) != 0;
           in_set = false;  // either we left, or a sender took us out and a delivery is coming
+          mail_due = !left;
         }
         if (left) {
-          if (lane == 0) __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          active = true;
+          if (leave_block_idle()) {
+            if (lane == 0) __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            publish();  // counted before anything this wave starts can end
+            enter(true);
+          }
           admit_tick = 0;  // the next pass admits
           continue;
         }
@@ -568,7 +685,10 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           break;
         }
         if (s == 0 && (!SERVE || stop)) break;
-        if (limited && gld(&g->done) >= P.limit) break;
+        if (limited && gld(&g->done) >= P.limit) {
+          if (leave_block_idle()) break;
+          continue;  // a ring just came in: its redexes go back to the global ring below
+        }
         if (wall_clock64() > t_end) {
           fail(L, ERR_TIMEOUT);
           break;
@@ -583,6 +703,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
                                            __HIP_MEMORY_SCOPE_AGENT);
             left = ((uniform(old) >> (gwave & 63)) & 1) != 0;
             in_set = false;  // either we left, or a sender took us out and a delivery is coming
+            mail_due = !left;
           }
           if (left) {
             u32 k = 0;
@@ -602,10 +723,13 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
             k = uniform(k);
             if (k > 0) {
               backoff = 1 + (gwave & 7);
-              active = true;
               if (TIMING) st[ST_CLAIMS]++;
               if (TIMING) st[ST_CLAIMED] += k;
-              claim_global(P, L, bag, top_c, k, lane, t_end);  // the rings are empty: k <= 64 fit
+              // (the claim counted this wave in S; a ring handed over
+              // meanwhile holds at most 64, so k <= 64 more fit)
+              if (leave_block_idle()) enter(true);
+              else if (lane == 0) __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              claim_global(P, L, bag, top_c, k, lane, t_end);
               __builtin_amdgcn_wave_barrier();
               continue;
             }
@@ -619,19 +743,16 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
         }
       }
       if (use_mbox) {
-        wave_sleep(MBOX_POLL);
+        idle_ticks = MBOX_POLL;
       } else {
-        wave_sleep(backoff);
+        idle_ticks = backoff;
         backoff = backoff < MAX_BACKOFF ? backoff * 2 + (gwave & 3) : MAX_BACKOFF - (gwave & 63);
       }
       continue;
     }
 
-    // ---- choose a ring: the fullest of the anni / comm / other rings if any
-    // holds redexes (they are cheap and release the work behind them, and
-    // definition calls meanwhile gather into fuller iterations), else the
-    // fullest definition-call ring; lowest index on ties
-    u32 key = lane < NCLS ? ((lane < CLS_CALL && my_n > 0) ? (1u << 24) : 0u) | (my_n << 4) | (15 - lane) : 0;
+    // ---- choose a ring
+    u32 key = lane < NCLS ? ring_key(lane, my_n) : 0;
     key = row0_max(key);
     const u32 c = admitting ? (u32)CLS_CALL : 15 - (key & 15);
     const u32 nc = (key >> 4) & 0xFFFFF;
@@ -666,7 +787,8 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
           if (t2 != b2) S_cache = spill_to_global(P, bag, &bot_c[cc], cc, t2 - b2, lane, b2, qerr);
         }
         if (qerr) fail(L, qerr);
-        if (lane == 0 && active) __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (lane == 0 && lds_add(&s_act, ~0u) == 1)
+          __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         active = false;
         break;
       }
@@ -677,18 +799,41 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     const u64 t_it = timing ? wall_clock64() : 0;
     if (TIMING) st[ST_BUSY_IT]++;
     const u32 nth = (lane - rot) & 63;  // this lane runs the nth-newest redex
-    bool has = nth < take;
+    u32 slot = ring_base(c) + ((top - 1 - nth) & (ring_cap(c) - 1)), total = take;
+    if (lane == c) my_top -= take;
+    if (P.fill && c >= CLS_CALL && !limited && !admitting) {
+      // batched nets: the free lanes run redexes of the other call rings.
+      // Fewer, longer passes: where there is work for every lane that is
+      // throughput (512 nets 197 -> 181 ms); a single net waits for its
+      // longest definition more often (bitonic 2^6 7.5 -> 9.8 ms), so there a
+      // pass keeps to one ring
+#pragma unroll
+      for (u32 q = CLS_CALL; q < NCLS; q++) {
+        const u32 nq = q == c ? 0 : lane_at(my_n, q), tq = nq < 64 - total ? nq : 64 - total;
+        if (tq) {
+          const u32 off = nth - total;
+          if (off < tq) slot = ring_base(q) + ((lane_at(my_top, q) - 1 - off) & (ring_cap(q) - 1));
+          if (lane == q) my_top -= tq;
+          total += tq;
+        }
+      }
+    }
+    bool has = nth < total;
     u64 ra = 0, rb = 0;
     if (has) {
-      const pair r = bag[ring_base(c) + ((top - 1 - nth) & (ring_cap(c) - 1))];
+      const pair r = bag[slot];
       ra = r.a;
       rb = r.b;
     }
-    rot = (rot + take) & 63;
+    rot = (rot + total) & 63;
     __builtin_amdgcn_wave_barrier();
-    if (lane == 0) top_c[c] = top - take;
+    if (lane < NCLS) top_c[lane] = my_top;
     __builtin_amdgcn_wave_barrier();
     const u64 t_in = timing ? wall_clock64() : 0;
+    // a wave woken inside its block is still in the idle set: its mailbox is
+    // read here and looked at after the tasks
+    u64 mail = 0;
+    if (use_mbox && (in_set || mail_due) && lane == 0) mail = gld(my_box);
     L.rw[RW_POPS] += has;
     run_tasks(L, c, has, ra, rb, boot, boot_def, boot_t0, np0);
     if (SERVE && (has || boot)) serve_account_deferred(L, L.pushed - 1u);
@@ -727,12 +872,63 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     }
     my_n = my_top - my_bot;
     n = row0_sum(my_n);
+    // ---- mail that came in meanwhile, once the rings have room for all of it
+    // (its count in S goes back: this block has one)
+    if (use_mbox && (in_set || mail_due) && n <= 64) {
+      const u64 k = uniform(mail);
+      if (k > 0 && k <= MBOX_PAIRS) {
+        take_mail(my_box, L, bag, top_c, (u32)k, lane, t_end);
+        if (lane == 0) __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        in_set = false;
+        mail_due = false;
+        my_top = lane < NCLS ? top_c[lane] : 0;
+        my_n = my_top - my_bot;
+        n += (u32)k;
+      }
+    }
+    // ---- idle waves of this block: each gets a whole ring, while this wave
+    // has another one for its next pass
+    // (batched nets, while the global ring holds work: fuller iterations are
+    // worth more than busier waves)
+    const bool share_ok = !(P.fill && (S_cache >> 32) > 0);
+    u32 rings = 0;  // those with redexes, but for the one to run next
+    if (share_ok) {
+      key = row0_max(lane < NCLS ? ring_key(lane, my_n) : 0);
+      rings = (u32)__ballot(lane < NCLS && my_n > 0) & ~(1u << (15 - (key & 15)));
+    }
+    if (rings) {
+      u32 sib = uniform(lds_get(&s_idle));
+      if (SERVE && sib) publish();  // the net's count of these redexes
+      while (sib && rings) {
+        const u32 t = (u32)__builtin_ctz(sib), r = (u32)__builtin_ctz(rings);
+        sib &= sib - 1;
+        u32 old = 0;
+        if (lane == 0) old = lds_and(&s_idle, ~(1u << t));
+        if (((uniform(old) >> t) & 1) == 0) continue;
+        rings &= rings - 1;
+        const u32 bot_r = lane_at(my_bot, r), n_r = lane_at(my_n, r), give = n_r < 64 ? n_r : 64;
+        if (lane < give) s_bag[t][ring_base(r) + lane] = bag[ring_base(r) + ((bot_r + lane) & (ring_cap(r) - 1))];
+        if (lane == r) {
+          my_bot += give;
+          my_n -= give;
+          bot_c[r] = my_bot;
+          s_top[t][r] = give;
+          s_bot[t][r] = 0;
+        }
+        n -= give;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0) {
+          (void)lds_add(&s_act, 1u);
+          lds_put(&s_given[t], 1u);
+        }
+      }
+    }
     key = lane < NCLS ? (my_n << 4) | (15 - lane) : 0;
     key = row0_max(key);
     const u32 sc = 15 - (key & 15);
     const u32 snc = key >> 4;
-    u32 active_waves = (u32)(S_cache & 0xFFFFFFFFu);
-    u32 idle_waves = P.total_waves > active_waves ? P.total_waves - active_waves : 0;
+    const u32 busy_waves = (u32)(S_cache & 0xFFFFFFFFu) * WAVES_PER_BLOCK;  // S counts blocks
+    u32 idle_waves = P.total_waves > busy_waves ? P.total_waves - busy_waves : 0;
     u32 queued = (u32)(S_cache >> 32);
     u32 spill = 0;
     if (snc > ring_cap(sc) * 3 / 4) spill = snc - ring_cap(sc) / 2;  // keep room for one iteration's pushes
@@ -742,47 +938,62 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     // MBOX_KEEP redexes hands the excess to one of them; keeping more makes
     // fuller iterations (batched mix: 29% faster keeping 256 than 80)
     if (use_mbox && idle_waves > 0 && n > mbox_keep && spill == 0) spill = snc < n - mbox_keep ? snc : n - mbox_keep;
-    const u32 spill0 = spill;
+    // with no idle wave left in this block, another ring goes to an idle wave
+    // elsewhere, too
+    bool share = false;
+    u32 from = sc;
+    if (share_ok && use_mbox && spill == 0 && rings && (u32)S_cache <= SHARE_BLOCKS && idle_waves > 0) {
+      share = true;
+      from = (u32)__builtin_ctz(rings);
+      spill = lane_at(my_n, from);
+    }
+    const u32 spill0 = share ? 0 : spill;
     if (spill && use_mbox && idle_waves > 0) {
-      // hand up to MBOX_PAIRS of the excess to one idle wave
+      // hand up to MBOX_PAIRS of the excess to one idle wave, by what this
+      // wave last saw of the idle set (idle_word: lane i holds word i)
       const u32 give = spill < MBOX_PAIRS ? spill : MBOX_PAIRS;
-      const u32 start = (gwave * 7u) % P.idle_words;
-      u32 wi = start + lane;
-      wi = wi >= P.idle_words ? wi - P.idle_words : wi;
-      const u64 w = lane < P.idle_words ? gld(&P.idle_bits[wi]) : 0;
-      const u64 ball = __ballot(w != 0);
+      const u32 first_word = (gwave * 7u) % P.idle_words;
+      if (!share) idle_word = lane < P.idle_words ? gld(&P.idle_bits[lane]) : 0;
+      const u64 ball = __ballot(lane < P.idle_words && idle_word != 0);
       if (ball) {
-        const u32 first = (u32)__builtin_ctzll(ball);
-        const u32 word = lane_at(wi, first);
-        const u64 bits = lane_at(w, first);
+        const u64 from_first = ball >> first_word << first_word;
+        const u32 word = (u32)__builtin_ctzll(from_first ? from_first : ball);
+        const u64 bits = lane_at(idle_word, word);
         const u32 r = gwave & 63;
         const u64 rot = (bits >> r) | (r ? bits << (64 - r) : 0);
         const u32 bit = ((u32)__builtin_ctzll(rot) + r) & 63;
-        u64 old = 0;
-        if (lane == 0)
+        // the receiver counts in S before it can start; both atomics are
+        // waited for together
+        u64 old = 0, s_old = 0;
+        if (lane == 0) {
+          s_old = __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           old = __hip_atomic_fetch_and(&P.idle_bits[word], ~(1ull << bit), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const bool got = ((uniform(old) >> bit) & 1) != 0;
-        const u32 target = word * 64 + bit;
-        if (got && target < P.total_waves) {
-          if (lane == 0) __hip_atomic_fetch_add(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          publish();  // the nodes these redexes reach, before the mailbox entries
-          u64 *box = P.mbox + (u64)target * MBOX_WORDS;
-          const u32 bot0 = lane_at(my_bot, sc);
+        }
+        publish();
+        old = uniform(old);
+        S_cache = uniform(s_old);
+        if (lane == word) idle_word = old & ~(1ull << bit);
+        if ((old >> bit) & 1) {
+          // pairs and count go out together: the receiver waits for every
+          // pair it reads to be there
+          u64 *box = P.mbox + (u64)(word * 64 + bit) * MBOX_WORDS;
+          const u32 bot0 = lane_at(my_bot, from);
           if (lane < give) {
-            const pair r = bag[ring_base(sc) + ((bot0 + lane) & (ring_cap(sc) - 1))];
-            gst(box + 16 + 2 * lane, r.a);
-            gst(box + 16 + 2 * lane + 1, r.b);
+            const pair p = bag[ring_base(from) + ((bot0 + lane) & (ring_cap(from) - 1))];
+            st16(box + 16 + 2 * lane, p.a, p.b);
           }
-          publish();
           if (lane == 0) {
             gst(box, (u64)give);
-            bot_c[sc] = bot0 + give;
+            bot_c[from] = bot0 + give;
           }
           if (TIMING) st[ST_SPILLS]++;
           if (TIMING) st[ST_SPILLED] += give;
           spill = 0;
+        } else if (lane == 0) {
+          __hip_atomic_fetch_sub(&g->S, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
       }
+      if (share) spill = 0;
     }
     if (spill) {
       const u64 t_sp = timing ? wall_clock64() : 0;

@@ -730,12 +730,13 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     // device: pending | root | tag | free ring | counters | words | base0 | len | gmap | inl
     const u64 inl_words = (u64)h->waves * 64 * SERVE_INL * 2;
     const u64 nsub = (u64)slots * SERVE_SUB;
-    const u64 words = (slots + 1) / 2 + 3 * (u64)slots + SV_WORDS + 2 * nsub + (nsub + 1) / 2 + (gmap_len + 1) / 2 +
+    const u64 pending_words = (u64)slots * PENDING_STRIDE / 2;
+    const u64 words = pending_words + 3 * (u64)slots + SV_WORDS + 2 * nsub + (nsub + 1) / 2 + (gmap_len + 1) / 2 +
                       inl_words + 64;
     hip_check(hipMalloc(&sv.dev, words * 8), "hipMalloc serving");
     u64 *w = sv.dev;
     u32 *pending = (u32 *)w;
-    w += (slots + 1) / 2;
+    w += pending_words;
     u64 *slot_root = w;
     w += slots;
     u64 *slot_tag = w;
@@ -768,7 +769,7 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     }
     h_ctl[SV_FREE_TAIL] = slots;
     h_ctl[SV_FREE_COUNT] = slots;
-    hip_check(hipMemset(pending, 0, (size_t)slots * 4), "init serving");
+    hip_check(hipMemset(pending, 0, pending_words * 8), "init serving");
     hip_check(hipMemcpy(free_ring, h_free.data(), (size_t)slots * 8, hipMemcpyHostToDevice), "init serving");
     hip_check(hipMemcpy(ctl, h_ctl.data(), SV_WORDS * 8, hipMemcpyHostToDevice), "init serving");
     hip_check(hipMemcpy(word, h_word.data(), nsub * 8, hipMemcpyHostToDevice), "init serving");
@@ -812,6 +813,7 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     P.serve = 1;
     P.serve_slots = slots;
     P.pending = pending;
+    P.sub_granules = (u32)sub_g;
     P.slot_root = slot_root;
     P.slot_tag = slot_tag;
     P.free_ring = free_ring;

@@ -195,7 +195,8 @@ struct Params {
   // Request and completion rings live in pinned host memory.
   u32 serve;
   u32 serve_slots;
-  u32 *pending;
+  u32 *pending;        // slot s: word s * PENDING_STRIDE
+  u32 sub_granules;    // granules of a slot's sub-arena
   u64 *slot_root;      // root cell of each slot's net
   u64 *slot_tag;       // the request's tag
   u64 *free_ring;      // slot + 1 entries (0: not yet written), serve_slots entries
@@ -220,8 +221,11 @@ enum : u32 { SH_REQ_TAIL = 0, SH_REQ_HEAD = 16, SH_DONE_READ = 32, SH_STOP = 48,
 // pending per lane).
 static const u32 SERVE_INL = 32;
 // A serving slot's arena is this many sub-arenas (consecutive, whole
-// granules each), taken from by the lanes of matching index.
+// granules each).
 static const u32 SERVE_SUB = 8;
+// The slots' counts of pending redexes stand on 128-byte lines of their own:
+// every task of a slot changes its count.
+static const u32 PENDING_STRIDE = 32;
 
 // Mailbox of a wave: a count word on its own 128-byte line, then up to
 // MBOX_PAIRS redex pairs handed to the wave by another wave (a zero word: not

@@ -232,10 +232,6 @@ DEV void lds_or(u32 *p, u32 v) { (void)__hip_atomic_fetch_or(p, v, __ATOMIC_RELA
 // register reads; sums and maxima over the lanes of row 0 (the ring classes,
 // NCLS <= 16) are four DPP row shifts.  Measured through LDS and then this
 // way: Church c2^c9, one busy wave, 5.38 -> 5.05 ms; bitonic 2^6 8.31 -> 8.19.
-DEV u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
-DEV u64 uniform(u64 v) { return (u64)uniform((u32)v) | (u64)uniform((u32)(v >> 32)) << 32; }
-DEV u32 lane_at(u32 v, u32 i) { return __builtin_amdgcn_readlane(v, i); }
-DEV u64 lane_at(u64 v, u32 i) { return (u64)lane_at((u32)v, i) | (u64)lane_at((u32)(v >> 32), i) << 32; }
 // The value n lanes below in the row of 16 (0 beyond its edge).
 template <u32 n>
 DEV u32 row_below(u32 v) { return __builtin_amdgcn_update_dpp(0, v, 0x110 + n, 0xF, 0xF, true); }
@@ -836,7 +832,7 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     if (use_mbox && (in_set || mail_due) && lane == 0) mail = gld(my_box);
     L.rw[RW_POPS] += has;
     run_tasks(L, c, has, ra, rb, boot, boot_def, boot_t0, np0);
-    if (SERVE && (has || boot)) serve_account_deferred(L, L.pushed - 1u);
+    if (SERVE) serve_account_deferred(L, has || boot);
     {
       const u64 dt = timing ? wall_clock64() - t_in : 0;
       if (TIMING) st[ST_INTERACT_TICKS] += dt;

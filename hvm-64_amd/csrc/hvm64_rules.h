@@ -16,6 +16,9 @@
 #define HVM_LDS_FAA(p, v) atomicAdd((p), (v))
 // True on any lane of the wave that is running.
 #define HVM_ANY(c) (__ballot(c) != 0)
+#define HVM_BALLOT(c) __ballot(c)
+// Bits of a ballot below this lane.
+#define HVM_BELOW(m) __builtin_amdgcn_mbcnt_hi((u32)((m) >> 32), __builtin_amdgcn_mbcnt_lo((u32)(m), 0u))
 // Pinned host memory (serving rings): system-scope accesses.
 #define HVM_LD_SYS(p) __hip_atomic_load((p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
 #define HVM_ST_SYS(p, v) __hip_atomic_store((p), (v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM)
@@ -41,6 +44,8 @@ typedef __attribute__((address_space(3))) unsigned long long lds_u64;
 #define HVM_CAS(p, e, v) __atomic_compare_exchange_n((p), (e), (v), false, __ATOMIC_RELAXED, __ATOMIC_RELAXED)
 #define HVM_LDS_FAA(p, v) __atomic_fetch_add((p), (v), __ATOMIC_RELAXED)
 #define HVM_ANY(c) (c)
+#define HVM_BALLOT(c) ((c) ? 1ull : 0ull)
+#define HVM_BELOW(m) ((void)(m), 0u)
 #define HVM_LD_SYS(p) __atomic_load_n((p), __ATOMIC_RELAXED)
 #define HVM_ST_SYS(p, v) __atomic_store_n((p), (v), __ATOMIC_RELAXED)
 #define HVM_FENCE_SYS() __atomic_thread_fence(__ATOMIC_RELEASE)
@@ -52,7 +57,17 @@ typedef unsigned long long lds_u64;
 
 namespace hvm {
 
-
+// Wave-wide values.  Lane 0's value (of the lanes running) and a lane at a
+// wave-uniform index.
+#if defined(__HIPCC__) || defined(__HIP__)
+DEV u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
+DEV u32 lane_at(u32 v, u32 i) { return __builtin_amdgcn_readlane(v, i); }
+#else
+DEV u32 uniform(u32 v) { return v; }
+DEV u32 lane_at(u32 v, u32) { return v; }
+#endif
+DEV u64 uniform(u64 v) { return (u64)uniform((u32)v) | (u64)uniform((u32)(v >> 32)) << 32; }
+DEV u64 lane_at(u64 v, u32 i) { return (u64)lane_at((u32)v, i) | (u64)lane_at((u32)(v >> 32), i) << 32; }
 
 static const u32 WAVES_PER_BLOCK = 4;
 // Every wave keeps its pending redexes in LDS, in one ring per rule class, so
@@ -387,8 +402,52 @@ DEV u32 net_of_port(const Params &P, u64 p, u32 dflt) {
     report_error(P.g, ERR_BADPTR, BAD_NET, p);
     return dflt;
   }
-  const u32 net = HVM_LD(&P.gmap[g]);
+  // (serving: the map never changes, so its words may come from the caches)
+  const u32 net = P.serve ? P.gmap[g] : HVM_LD(&P.gmap[g]);
   return net < P.n_nets ? net : dflt;
+}
+
+// Serving: the lanes of a wave that take nodes together and are on the same
+// slot take them with one atomic add: exactly `need` nodes each, side by
+// side.  (Every serving lane takes at nearly every task, since its slot may
+// restart in between; with an atomic per lane the words of a few dozen slots
+// were the hottest lines of the launch.)  A slot's arena is SERVE_SUB
+// sub-arenas; the lane that adds goes through them in turn.
+DEV void arena_room_serve(Lane &L, u32 need) {
+  const Params &P = *L.P;
+  const u64 len = (u64)P.sub_granules << P.gran_shift;
+  for (u64 todo = HVM_BALLOT(true); todo;) {
+    const u32 lead = (u32)__builtin_ctzll(todo);
+    const u32 net = lane_at(L.cur_net, lead);
+    const bool mine = L.cur_net == net;
+    const u64 same = HVM_BALLOT(mine);
+    u32 sum = 0, before = 0;
+    for (u32 b = 0; HVM_ANY(need >> b != 0); b++) {
+      const u64 m = HVM_BALLOT(mine && ((need >> b) & 1));
+      sum += (u32)__builtin_popcountll(m) << b;
+      before += HVM_BELOW(m) << b;
+    }
+    // (a full sub-arena gives its add back and the next one is tried)
+    const u32 first = lane_at(L.rw[RW_POPS], lead) + lead;
+    u64 w = 0;
+    bool fits = false;
+    for (u32 k = 0; k < SERVE_SUB && !fits; k++) {
+      u64 *const word = &P.arena_word[net * SERVE_SUB + ((first + k) & (SERVE_SUB - 1))];
+      if (L.lane_id == lead) w = HVM_FAA(word, (u64)sum);
+      w = lane_at(w, lead);
+      fits = (w & 0xFFFFFFFFull) + sum <= len;
+      if (!fits && L.lane_id == lead) HVM_FAA(word, (u64)0 - sum);
+    }
+    if (mine) {
+      L.a_pos = ((w >> 32) << P.gran_shift) + (w & 0xFFFFFFFFull) + before;
+      L.a_end = L.a_pos + need;
+      if (!fits) {
+        fail(L, ERR_OOM, OOM_POOL);
+        L.a_end = L.a_pos;
+      }
+    }
+    todo &= ~same;
+  }
 }
 
 // Makes room for `need` consecutive nodes of the running task's net.  Right
@@ -396,6 +455,10 @@ DEV u32 net_of_port(const Params &P, u64 p, u32 dflt) {
 // another net's, and the rest of a chunk would stay unused); while it stays
 // on one net each take doubles, up to the chunk.
 DEV void arena_room(Lane &L, u32 need) {
+  if (L.serve) {
+    arena_room_serve(L, need);
+    return;
+  }
   const bool same = L.a_net == L.cur_net;
   if (same && L.a_pos + need <= L.a_end) return;
   const Params &P = *L.P;
@@ -403,12 +466,7 @@ DEV void arena_room(Lane &L, u32 need) {
   t = t > P.arena_chunk ? P.arena_chunk : t;
   L.a_take = t;
   const u32 net = L.cur_net;
-  // serving: a slot's arena is SERVE_SUB sub-arenas, each with its own word,
-  // a lane taking from the one of its lane index (a serving lane takes at
-  // nearly every task, and one word per slot was hammered by every lane on
-  // that slot)
-  const u32 wi = L.serve ? net * SERVE_SUB + (L.lane_id & (SERVE_SUB - 1)) : net;
-  const ArenaChunk c = arena_take(&P.arena_word[wi], P.arena_base0[wi], P.arena_len[wi], P.refill_granules,
+  const ArenaChunk c = arena_take(&P.arena_word[net], P.arena_base0[net], P.arena_len[net], P.refill_granules,
                                   P.gran_shift, P.pool_next, P.pool_end, P.gmap, net, P.ov_next, P.ov_end,
                                   need > t ? need : t);
   L.a_net = L.cur_net;
@@ -590,7 +648,7 @@ DEV void push_global(u64 *queue, u64 qmask, Globals *g, u64 a, u64 b) {
 DEV void global_push1(Lane &L, u64 a, u64 b) {
   // serving: a redex in the global ring can be taken and finished by another
   // wave before this task ends, so it is counted for its net at once
-  if (L.serve) HVM_FAA(&L.P->pending[L.cur_net], 1u);
+  if (L.serve) HVM_FAA(&L.P->pending[(u64)L.cur_net * PENDING_STRIDE], 1u);
   push_global(L.P->queue, L.P->qmask, L.P->g, a, b);
 }
 
@@ -1327,11 +1385,28 @@ DEV void serve_complete(Lane &L, u32 s) {
 // another wave first retires the wave's memory operations (this one too),
 // and the wave pops its own rings only after serve_settle, so no consumer's
 // decrement can overtake it.
-DEV void serve_account_deferred(Lane &L, u32 delta) {
-  L.acct_delta = delta;
-  if (delta == 0) return;
-  L.acct_net = L.cur_net;
-  L.acct_old = HVM_FAA(&L.P->pending[L.cur_net], delta);
+// One atomic per slot and wave: the changes of the lanes on a slot are summed,
+// and the first of those lanes sends the sum and looks at it later (an atomic
+// per lane, all slots' words on a few lines, held every iteration up: 128
+// requests on 32 slots, 350 ms; with this and arena_room_serve 136 ms).  All lanes call it; `ran`: the lane ran a
+// task or a boot.
+DEV void serve_account_deferred(Lane &L, bool ran) {
+  L.acct_delta = 0;
+  const u32 delta = L.pushed;  // of the redexes put in rings; one was consumed by each lane
+  for (u64 todo = HVM_BALLOT(ran); todo;) {
+    const u32 lead = (u32)__builtin_ctzll(todo);
+    const u32 net = lane_at(L.cur_net, lead);
+    const u64 same = HVM_BALLOT(ran && L.cur_net == net);
+    u32 sum = 0u - (u32)__builtin_popcountll(same);
+    for (u32 b = 0; HVM_ANY(delta >> b != 0); b++)
+      sum += (u32)__builtin_popcountll(HVM_BALLOT(ran && L.cur_net == net && ((delta >> b) & 1))) << b;
+    if (L.lane_id == lead && sum != 0) {
+      L.acct_delta = sum;
+      L.acct_net = net;
+      L.acct_old = HVM_FAA(&L.P->pending[(u64)net * PENDING_STRIDE], sum);
+    }
+    todo &= ~same;
+  }
 }
 
 DEV void serve_settle(Lane &L) {
@@ -1429,7 +1504,7 @@ DEV u64 serve_boot(Lane &L, u32 s, u64 tag, u32 &np) {
   const Params &P = *L.P;
   L.cur_net = s;
   L.a_net = NO_NET;
-  HVM_FAA(&P.pending[s], 1u);
+  HVM_FAA(&P.pending[(u64)s * PENDING_STRIDE], 1u);
   HVM_ST(&P.slot_tag[s], tag);
   u64 m[2];
   alloc_nodes(L, 2, m);

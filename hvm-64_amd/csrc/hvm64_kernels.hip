@@ -894,7 +894,9 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     }
     if (rings) {
       u32 sib = uniform(lds_get(&s_idle));
-      if (SERVE && sib) publish();  // the net's count of these redexes
+      // the nodes these redexes reach (a lane of this wave may read them with
+      // their stores under way, another wave not); serving: their net's count
+      if (sib) publish();
       while (sib && rings) {
         const u32 t = (u32)__builtin_ctz(sib), r = (u32)__builtin_ctz(rings);
         sib &= sib - 1;

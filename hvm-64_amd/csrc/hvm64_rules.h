@@ -123,11 +123,14 @@ DEV u64 *hw(Lane &L, u64 addr);
 // gfx940 and later need two wait states before a VALU instruction may
 // overwrite the data registers of a store wider than 64 bits; the compiler
 // does not insert them after inline asm, so the asm ends with `s_nop 1`.
+// No memory clobber here and in the loads below: they are volatile, so they
+// keep their order among themselves and to publish(), and LDS accesses may
+// be scheduled around them.
 DEV void st16(u64 *p, u64 w0, u64 w1) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef u64 u64x2 __attribute__((ext_vector_type(2)));
   const u64x2 d = {w0, w1};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(d) : "memory");
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(d));
 #else
   HVM_ST(p, w0);
   HVM_ST(p + 1, w1);
@@ -142,7 +145,8 @@ DEV u64 var_port(u64 cell) { return mkport(T_VAR, 0, cell); }
 DEV u64 wire_port(u64 cell) { return mkport(T_RED, 0, cell); }
 // Endpoints are stored as Var ports; the Red tag only marks trg registers
 // that the interpreter may resolve (the reference's Trg::wire, linker.rs:233-281).
-DEV u64 norm_endpoint(u64 p) { return is_endpoint(p) ? (paddr(p) | T_VAR) : p; }
+// (An endpoint's label is 0: only the tag changes.)
+DEV u64 norm_endpoint(u64 p) { return is_endpoint(p) ? (p | T_VAR) : p; }
 
 // ---------------------------------------------------------------------------
 // per-lane state
@@ -233,7 +237,7 @@ DEV u64 *hw(Lane &L, u64 addr) {
   const u64 off = addr - HVM_HEAP_OFF;
   const bool out = off >= P.heap_words * 8;
   L.bad = out ? addr : L.bad;
-  return P.heap + ((out ? DUMP_WORD * 8 : off) >> 3);
+  return (u64 *)((char *)P.heap + (out ? DUMP_WORD * 8 : off & ~7ull));
 }
 DEV u64 ld(Lane &L, u64 addr) { return HVM_LD(hw(L, addr)); }
 DEV void st(Lane &L, u64 addr, u64 v) { HVM_ST(hw(L, addr), v); }
@@ -544,8 +548,7 @@ DEV void ld16x2(const u64 *p, const u64 *q, u64 &p0, u64 &p1, u64 &q0, u64 &q1) 
   u64x2 dp, dq;
   asm volatile("global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
                : "=&v"(dp), "=&v"(dq)
-               : "v"(p), "v"(q)
-               : "memory");
+               : "v"(p), "v"(q));
   p0 = dp.x;
   p1 = dp.y;
   q0 = dq.x;
@@ -561,7 +564,7 @@ DEV void ld16(const u64 *p, u64 &p0, u64 &p1) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef u64 u64x2 __attribute__((ext_vector_type(2)));
   u64x2 dp;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=v"(dp) : "v"(p) : "memory");
+  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=v"(dp) : "v"(p));
   p0 = dp.x;
   p1 = dp.y;
 #else
@@ -766,7 +769,8 @@ DEV void flush_links(Lane &L, u32 &np) {
       red &= red - 1;
       redux(L, a, b);
     }
-    publish();
+    // (the nodes these ports lead to; the later rounds' are the other side's)
+    if (round == 0) publish();
     u64 o[4];
 #pragma unroll
     for (u32 j = 0; j < 4; j++) {
@@ -790,25 +794,30 @@ DEV void flush_links(Lane &L, u32 &np) {
 // caller owns the endpoint, so once a cell holds a port the cell is ours to
 // free.
 DEV u64 follow(Lane &L, u64 p, bool go) {
-  for (u32 hop = 0; go; hop++) {
-    if (hop > MAX_CHAIN) {
-      fail(L, ERR_BADPTR, BAD_RESOLVE);
-      return P_ERA;
-    }
-    u64 *const w = hw(L, paddr(p));
-    const u64 v = HVM_LD(w);
-    go = v != P_NONE;
+  for (u32 hop = 0; HVM_ANY(go); hop++) {
     if (go) {
-      if (!L.arenas) HVM_ST(w, P_FREE);
-      p = v;
-      go = is_endpoint(v);
+      u64 *const w = hw(L, paddr(p));
+      const u64 v = HVM_LD(w);
+      go = v != P_NONE;
+      if (go) {
+        if (!L.arenas) HVM_ST(w, P_FREE);
+        p = v;
+        go = is_endpoint(v);
+      }
+    }
+    if (hop >= MAX_CHAIN) {
+      if (go) {
+        fail(L, ERR_BADPTR, BAD_RESOLVE);
+        p = P_ERA;
+      }
+      break;
     }
   }
   return p;
 }
 DEV u64 resolve(Lane &L, u64 p) { return follow(L, p, is_endpoint(p)); }
 
-DEV u64 as_wire(u64 p) { return is_endpoint(p) ? wire_port(paddr(p)) : p; }
+DEV u64 as_wire(u64 p) { return is_endpoint(p) ? p & ~(u64)T_VAR : p; }
 
 // operate_binary, whose unsigned operations that neither divide nor shift
 // are computed here: they are nearly all of a program's, and the general
@@ -1092,11 +1101,6 @@ DEV void run_template(Lane &L, Interp &I, u32 off) {
   }
 }
 
-// The instruction kinds in three groups, each run by a loop of its own
-// (interp_run): the kinds that match the argument or make registers, the
-// links, and I_TEMPLATE.
-DEV bool is_link_kind(u32 kind) { return kind == I_LINK || kind == I_LINKCONST || kind == I_LINKT; }
-
 // One Ctr / Op / OpNum / Switch / Const / Wires instruction
 // (instruction.rs:110-210).  Every lane goes through the same sequence (read
 // the trg, follow it, take the node, take fresh nodes, write two registers),
@@ -1116,19 +1120,26 @@ DEV void exec_step(Lane &L, Interp &I, u64 w0, u64 w1, u32 &np) {
   u64 x = 0, y = 0;
   if (match) take(L, p, x, y);
   L.rw[RW_ANNI] += match;
-  const u32 need = match ? 0 : ctr ? 2 : other_need(kind, p);
-  u64 m[3] = {0, 0, 0};
-  if (need) alloc_nodes(L, need, m);
   if (ctr) {
     if (!match) {  // instruction.rs:126-131
+      u64 m[2];
+      alloc_nodes(L, 2, m);
       st2_new(P, m[0], P_NONE, P_NONE);
-      st2_new(P, m[1], var_port(m[0]), var_port(m[0] + 8));
+      x = var_port(m[0]);
+      y = var_port(m[0] + 8);
+      st2_new(P, m[1], x, y);
       push_link(L, np, p, mkport(T_CTR, lab, m[1]));
     }
-    t_set(I, b, match ? as_wire(x) : var_port(m[0]));
-    t_set(I, c, match ? as_wire(y) : var_port(m[0] + 8));
-  } else {
-    exec_other(L, I, w0, w1, p, m, np);
+    t_set(I, b, match ? as_wire(x) : x);
+    t_set(I, c, match ? as_wire(y) : y);
+  }
+  if (HVM_ANY(!ctr)) {
+    if (!ctr) {
+      u64 m[3] = {0, 0, 0};
+      const u32 need = other_need(kind, p);
+      if (need) alloc_nodes(L, need, m);
+      exec_other(L, I, w0, w1, p, m, np);
+    }
   }
 }
 
@@ -1204,28 +1215,31 @@ DEV void fetch(const Lane &L, const Interp &I, u64 &w0, u64 &w1) {
 // lanes go through once; an interpreted program, whose links stand among its
 // patterns, goes round again.
 DEV void interp_run(Lane &L, Interp &I, u32 &np) {
+  const u32 LINKS = 1u << I_LINK | 1u << I_LINKCONST | 1u << I_LINKT;
   HVM_SETTLE_LOADS();
   u64 w0 = 0, w1 = 0;
-  while (I.left > 0 && np < LINK_CAP) {
+  u32 kb = 0;  // bit of the instruction that ended the loop
+  while ((I.left > 0) & (np < LINK_CAP)) {
     fetch(L, I, w0, w1);
-    const u32 kind = (u32)(w0 & 0xFF);
-    if (kind == I_TEMPLATE || is_link_kind(kind)) break;
+    kb = 1u << (w0 & 0x1F);
+    if (kb & (LINKS | 1u << I_TEMPLATE)) break;
     exec_step(L, I, w0, w1, np);
     I.ipw += 2;
     I.left -= 1;
   }
-  if (I.left > 0 && np < LINK_CAP && (u32)(w0 & 0xFF) == I_TEMPLATE) {
+  if ((I.left > 0) & (np < LINK_CAP) & ((kb >> I_TEMPLATE) & 1)) {
     run_template(L, I, (u32)w1);
     I.ipw += 2;
     I.left -= 1;
   }
-  while (I.left > 0 && np < LINK_CAP) {
+  while ((I.left > 0) & (np < LINK_CAP)) {
     fetch(L, I, w0, w1);
-    const u32 kind = (u32)(w0 & 0xFF);
-    if (!is_link_kind(kind)) break;
-    const u64 t_a = t_get(I, (u32)(w0 >> 16) & 0xFFFF);
-    push_link(L, np, t_a,
-              kind == I_LINK ? t_get(I, (u32)(w0 >> 32) & 0xFFFF) : kind == I_LINKT ? tspec(I, w1) : w1);
+    kb = 1u << (w0 & 0x1F);
+    if (!(kb & LINKS)) break;
+    const u64 t_a = t_get(I, (u32)(w0 >> 16) & 0xFFFF), t_b = t_get(I, (u32)(w0 >> 32) & 0xFFFF);
+    u64 v = (kb >> I_LINK) & 1 ? t_b : w1;
+    if (HVM_ANY((kb >> I_LINKT) & 1)) v = (kb >> I_LINKT) & 1 ? tspec(I, w1) : v;
+    push_link(L, np, t_a, v);
     I.ipw += 2;
     I.left -= 1;
   }
@@ -1491,7 +1505,6 @@ DEV void run_tasks(Lane &L, u32 cls, bool has, u64 a, u64 b, bool booting, u32 d
     cls = CLS_CALL;
     booting = false;
   }
-  publish();
 }
 
 // Serving: sets a lane up to boot a request into free slot s as Net::boot +

@@ -19,6 +19,9 @@ namespace hvm {
 hipError_t launch_fill(u64 *words, u64 n, u64 value, hipStream_t st);
 hipError_t launch_exec(const Params &P, u32 def, u64 t0, u32 count_dref, hipStream_t st);
 hipError_t launch_expand(const Params &P, u64 old_root_cell, hipStream_t st);
+hipError_t launch_prepare(const Params &P, hipStream_t st);
+hipError_t launch_mirror(const Params &P, hipStream_t st);
+hipError_t launch_reset(const Params &P, u64 q0, u64 q1, hipStream_t st);
 hipError_t launch_reduce(const Params &P, u32 blocks, hipStream_t st);
 hipError_t launch_boot_batch(const Params &P, u32 n, const u32 *defs, u64 *roots, u32 max_blocks, hipStream_t st);
 hipError_t launch_expand_batch(const Params &P, u32 n, u64 *roots, u32 max_blocks, hipStream_t st);
@@ -92,6 +95,12 @@ struct hvm_gpu {
   u32 idle_words = 0;
   Globals last{};
   double last_ms = 0;
+  // pinned host memory the kernels write: the control block, then short
+  // readback results; its device address
+  u64 *pin = nullptr, *pin_dev = nullptr;
+  u64 *d_net = nullptr;     // the code of hvm_gpu_encode_net_text's net
+  u64 d_net_cap = 0;        // words
+  bool ring_unknown = true; // the global ring may hold words outside [q_head, q_tail)
   // the serving launch (hvm_gpu_serve_start .. _stop)
   struct Serve {
     bool running = false;
@@ -134,6 +143,11 @@ void dfree(T *&p) {
   p = nullptr;
 }
 
+const u64 GLOBALS_WORDS = sizeof(Globals) / 8;
+// Readback results up to this many words reach the host with the launch
+// itself; longer ones are copied after it.
+const u64 RB_HOST_WORDS = 4096;
+
 Params make_params(hvm_gpu *h, u64 limit) {
   Params P{};
   P.heap = h->heap;
@@ -153,6 +167,9 @@ Params make_params(hvm_gpu *h, u64 limit) {
   P.queue = h->queue;
   P.qmask = h->qslots - 1;
   P.g = h->g;
+  P.g_host = h->pin_dev;
+  P.rb_host = h->pin_dev + GLOBALS_WORDS;
+  P.rb_host_cap = RB_HOST_WORDS;
   P.ndefs = h->ndefs;
   P.trg_slots = h->trg_slots;
   P.total_waves = h->waves;
@@ -173,9 +190,12 @@ Params make_params(hvm_gpu *h, u64 limit) {
   return P;
 }
 
-void sync_globals(hvm_gpu *h) {
+// Waits for the stream and takes over the control block, which the last
+// kernel has copied to the host (mirrored) or a kernel of its own does.
+void sync_globals(hvm_gpu *h, bool mirrored = false) {
+  if (!mirrored) hip_check(launch_mirror(make_params(h, ~0ull), h->stream), "launch mirror");
   hip_check(hipStreamSynchronize(h->stream), "kernel");
-  hip_check(hipMemcpy(&h->last, h->g, sizeof(Globals), hipMemcpyDeviceToHost), "read globals");
+  std::memcpy(&h->last, h->pin, sizeof(Globals));
   if (h->last.err) {
     u32 e = h->last.err;
     int code = e == ERR_OOM ? HVM_E_OOM
@@ -215,13 +235,13 @@ void ensure_trg(hvm_gpu *h, u32 slots) {
 
 // The device trusts the book's instructions (no per-step checks), so every
 // operand register index is checked here against its definition's size.
-void validate_book(const hvm_gpu *h) {
-  for (size_t i = 0; i < h->defs_host.size(); i++) {
-    const DefRec &d = h->defs_host[i];
-    if (d.nslots < 1 || (u64)d.ioff + d.ilen > h->instrs_host.size() / 2)
+void validate_book(const std::vector<DefRec> &defs, const std::vector<u64> &instrs) {
+  for (size_t i = 0; i < defs.size(); i++) {
+    const DefRec &d = defs[i];
+    if (d.nslots < 1 || (u64)d.ioff + d.ilen > instrs.size() / 2)
       throw Error(HVM_E_ARG, "book: definition " + std::to_string(i) + " is malformed");
     for (u32 k = 0; k < d.ilen; k++) {
-      u64 w0 = h->instrs_host[2 * ((u64)d.ioff + k)], w1 = h->instrs_host[2 * ((u64)d.ioff + k) + 1];
+      u64 w0 = instrs[2 * ((u64)d.ioff + k)], w1 = instrs[2 * ((u64)d.ioff + k) + 1];
       u32 kind = (u32)(w0 & 0xFF);
       u32 a = (u32)(w0 >> 16) & 0xFFFF, b = (u32)(w0 >> 32) & 0xFFFF, c = (u32)(w0 >> 48);
       u32 d4 = kind == I_WIRES ? (u32)(w1 & 0xFFFF) : 0;
@@ -232,7 +252,7 @@ void validate_book(const hvm_gpu *h) {
 }
 
 void upload_book(hvm_gpu *h) {
-  validate_book(h);
+  validate_book(h->defs_host, h->instrs_host);
   // The device book: the definitions' own instructions, then their compiled
   // programs and templates (hvm64_defcomp.cpp).
   hvm64::DeviceBook b = hvm64::build_device_book(h->defs_host, h->instrs_host);
@@ -265,19 +285,26 @@ void upload_book(hvm_gpu *h) {
 // net: a ring's first lap overwrites its slots without reading them, and
 // later laps only reuse slots whose words read FREE, so words left by a
 // previous net are either overwritten or skipped, never read as live.
+// The control block, the rings, the idle set and the mailboxes.  The global
+// redex ring (1 GiB) is cleared where it may hold redexes: every redex taken
+// from it leaves zeros, so after a reduction that ended well that is
+// [q_head, q_tail), usually nothing; after an error, all of it.  (Clearing it
+// all took 170 us of every Net::new, a quarter of a small program's run.)
+void clear_state(hvm_gpu *h) {
+  const bool all = h->ring_unknown || h->last.err != 0 || h->last.q_tail - h->last.q_head > h->qslots;
+  hip_check(launch_reset(make_params(h, ~0ull), all ? 0 : h->last.q_head, all ? h->qslots : h->last.q_tail, h->stream),
+            "reset");
+  hip_check(hipStreamSynchronize(h->stream), "reset");
+  h->last = Globals{};
+  h->ring_unknown = false;
+}
+
 void reset_net(hvm_gpu *h, bool fill) {
   fill = fill || h->heap_dirty;
   h->heap_dirty = false;
   if (fill) hip_check(launch_fill(h->heap, h->heap_words, P_FREE, h->stream), "fill heap");
-  hip_check(launch_fill(h->queue, h->qslots * 2, 0, h->stream), "clear ring");
-  Globals g0{};
-  hip_check(hipMemsetAsync(h->alloc_pos, 0, (size_t)h->waves * 64 * sizeof(u64), h->stream), "clear rings");
-  hip_check(hipMemcpyAsync(h->g, &g0, sizeof(Globals), hipMemcpyHostToDevice, h->stream), "init globals");
-  u64 none = P_NONE;
-  hip_check(hipMemcpyAsync(h->heap + ROOT0_WORD, &none, sizeof(u64), hipMemcpyHostToDevice, h->stream), "root");
+  clear_state(h);
   h->root_cell = HVM_HEAP_OFF + ROOT0_WORD * 8;
-  hip_check(hipStreamSynchronize(h->stream), "reset");
-  h->last = g0;
 }
 
 // Run the persistent reduction kernel with a redex budget.
@@ -285,15 +312,12 @@ void reset_net(hvm_gpu *h, bool fill) {
 // ring holds the excess, a wave whose rings run low claims from the global
 // ring without going idle first (fuller iterations; a single net, with many
 // idle waves, gains nothing from it).
-void run_reduce(hvm_gpu *h, u64 limit, bool fill = false) {
+// `prepared`: a kernel on the stream has cleared what the reduction starts
+// from (prepare_reduce).
+void run_reduce(hvm_gpu *h, u64 limit, bool fill = false, bool prepared = false) {
   Params P = make_params(h, limit);
   P.fill = fill ? 1 : 0;
-  u64 zero = 0;
-  u64 zst[ST_SLOTS] = {};
-  hip_check(hipMemcpyAsync(&h->g->done, &zero, sizeof(u64), hipMemcpyHostToDevice, h->stream), "budget");
-  hip_check(hipMemcpyAsync(h->g->st, zst, sizeof(zst), hipMemcpyHostToDevice, h->stream), "stats");
-  hip_check(hipMemsetAsync(h->idle_bits, 0, (size_t)h->idle_words * 8, h->stream), "clear idle set");
-  hip_check(hipMemsetAsync(h->mbox, 0, (size_t)h->waves * MBOX_WORDS * 8, h->stream), "clear mailboxes");
+  if (!prepared) hip_check(launch_prepare(P, h->stream), "launch prepare");
   hip_check(hipEventRecord(h->ev0, h->stream), "event");
   hip_check(launch_reduce(P, h->blocks, h->stream), "launch reduce");
   hip_check(hipEventRecord(h->ev1, h->stream), "event");
@@ -310,10 +334,8 @@ void run_reduce(hvm_gpu *h, u64 limit, bool fill = false) {
 std::string readback(hvm_gpu *h, u64 root_cell, bool with_redexes = false) {
   u64 q_head = 0, q_tail = 0;
   if (with_redexes) {
-    Globals g;
-    hip_check(hipMemcpy(&g, h->g, sizeof(Globals), hipMemcpyDeviceToHost), "read globals");
-    q_head = g.q_head;
-    q_tail = std::max(g.q_head, g.q_tail);
+    q_head = h->last.q_head;
+    q_tail = std::max(h->last.q_head, h->last.q_tail);
     if (q_tail - q_head > h->qslots) throw Error(HVM_E_READBACK, "readback: redex ring inconsistent");
   }
   for (;;) {
@@ -328,7 +350,7 @@ std::string readback(hvm_gpu *h, u64 root_cell, bool with_redexes = false) {
               "launch readback");
     hip_check(hipStreamSynchronize(h->stream), "readback");
     Globals g;
-    hip_check(hipMemcpy(&g, h->g, sizeof(Globals), hipMemcpyDeviceToHost), "read globals");
+    std::memcpy(&g, h->pin, sizeof(Globals));
     if (g.err == ERR_READBACK && g.err_info == 1 && h->rb_cap < (1ull << 31)) {
       u32 zero = 0;
       hip_check(hipMemcpy(&h->g->err, &zero, sizeof(u32), hipMemcpyHostToDevice), "clear err");
@@ -339,10 +361,12 @@ std::string readback(hvm_gpu *h, u64 root_cell, bool with_redexes = false) {
     }
     if (g.err) throw Error(HVM_E_READBACK, "readback: malformed net");
     std::vector<u64> stream(g.result);
-    if (g.result)
+    if (g.result > RB_HOST_WORDS)
       hip_check(hipMemcpy(stream.data(), h->d_rb_out, g.result * sizeof(u64), hipMemcpyDeviceToHost), "copy readback");
+    else
+      std::memcpy(stream.data(), h->pin + GLOBALS_WORDS, g.result * sizeof(u64));
     std::string text;
-    hvm64::with_big_stack([&] {
+    auto print = [&] {
       size_t pos = 0;
       std::map<u64, u64> vars;
       u64 next = 0;
@@ -352,7 +376,10 @@ std::string readback(hvm_gpu *h, u64 root_cell, bool with_redexes = false) {
         const std::string b = hvm64::readback_text(h->host, stream, pos, vars, next);
         text += "\n  & " + a + " ~ " + b;
       }
-    });
+    };
+    // a tree's depth is at most its size: a short one needs no stack of its own
+    if (stream.size() <= 512) print();
+    else hvm64::with_big_stack(print);
     return text;
   }
 }
@@ -787,13 +814,7 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     sv.req = sv.host + SH_WORDS;
     sv.done = sv.req + 2 * rq;
     // a clean control block, idle set, mailboxes and global ring
-    hip_check(launch_fill(h->queue, h->qslots * 2, 0, h->stream), "clear ring");
-    hip_check(hipMemsetAsync(h->idle_bits, 0, (size_t)h->idle_words * 8, h->stream), "clear idle set");
-    hip_check(hipMemsetAsync(h->mbox, 0, (size_t)h->waves * MBOX_WORDS * 8, h->stream), "clear mailboxes");
-    Globals g0{};
-    hip_check(hipMemcpyAsync(h->g, &g0, sizeof(Globals), hipMemcpyHostToDevice, h->stream), "init globals");
-    hip_check(hipStreamSynchronize(h->stream), "init serving");
-    h->last = g0;
+    clear_state(h);
     h->heap_dirty = true;
     Params P = make_params(h, ~0ull);
     P.fill = 1;
@@ -960,6 +981,11 @@ int hvm_gpu_open_grid(int device, uint64_t heap_bytes, uint32_t max_blocks, hvm_
     hip_check(hipMalloc(&h->idle_bits, (size_t)h->idle_words * 8), "hipMalloc idle set");
     hip_check(hipMalloc(&h->mbox, (size_t)h->waves * MBOX_WORDS * 8), "hipMalloc mailboxes");
     hip_check(hipMalloc(&h->g, sizeof(Globals)), "hipMalloc globals");
+    hip_check(hipHostMalloc((void **)&h->pin, (GLOBALS_WORDS + RB_HOST_WORDS) * 8,
+                            hipHostMallocMapped | hipHostMallocCoherent),
+              "hipHostMalloc results");
+    std::memset(h->pin, 0, (GLOBALS_WORDS + RB_HOST_WORDS) * 8);
+    hip_check(hipHostGetDevicePointer((void **)&h->pin_dev, h->pin, 0), "results' device address");
     // Global redex ring: 2^26 slots (1 GiB).  A massively parallel net keeps
     // about (lanes x recursion depth) redexes pending; the LDS rings hold
     // 256 per wave and the rest waits here.
@@ -1004,6 +1030,8 @@ void hvm_gpu_close(hvm_gpu *h) {
   dfree(h->d_trg);
   dfree(h->d_rb_out);
   dfree(h->d_rb_stack);
+  dfree(h->d_net);
+  if (h->pin) (void)hipHostFree(h->pin);
   if (h->ev0) (void)hipEventDestroy(h->ev0);
   if (h->ev1) (void)hipEventDestroy(h->ev1);
   if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -1107,7 +1135,7 @@ int hvm_gpu_pre_reduce(hvm_gpu *h, const char *book_text, const char *const *nam
       reset_net(h, false);
       Params P = make_params(h, ~0ull);
       hip_check(launch_exec(P, h->host.def_id(name), mkport(T_VAR, 0, h->root_cell), 1, h->stream), "launch boot");
-      sync_globals(h);
+      sync_globals(h, true);
       // reduce(limit) interacts once before it compares (net.rs:41-52)
       run_reduce(h, std::max<u64>(max_rwts, 1));
       for (int k = 0; k < 5; k++) total[k] += h->last.rw[k];
@@ -1124,6 +1152,7 @@ int hvm_gpu_pre_reduce(hvm_gpu *h, const char *book_text, const char *const *nam
       if (gl.captured_n) {
         const u64 nt = tail + gl.captured_n;
         hip_check(hipMemcpy(&h->g->q_tail, &nt, 8, hipMemcpyHostToDevice), "captured redexes");
+        h->last.q_tail = nt;
       }
       std::string text = readback(h, h->root_cell, true);
       hvm64::with_big_stack([&] {
@@ -1279,7 +1308,7 @@ int hvm_gpu_boot(hvm_gpu *h, uint32_t def_id) {
     if (def_id >= h->ndefs) throw Error(HVM_E_ARG, "no such definition");
     Params P = make_params(h, ~0ull);
     hip_check(launch_exec(P, def_id, mkport(T_VAR, 0, h->root_cell), 1, h->stream), "launch boot");
-    sync_globals(h);
+    sync_globals(h, true);
   });
 }
 
@@ -1292,38 +1321,52 @@ int hvm_gpu_encode_net_text(hvm_gpu *h, const char *net_text) {
       hvm64::Net net = hvm64::parse_net(arena, net_text);
       code = h->host.encode(arena, net);
     });
-    // Append the net's code as a temporary definition after the book.
+    // The net's code is a book of one definition, executed from a buffer of
+    // its own: the device's book stays as it is (putting the net behind the
+    // book and taking it out again uploaded the book twice, 10 allocations).
     DefRec r{};
-    r.ioff = (u32)(h->instrs_host.size() / 2);
     r.ilen = code.ninstr();
     r.nslots = code.nslots;
-    r.labs_off = 0;
-    r.labs_words = 0;
-    r.min_safe = 0;
-    std::vector<DefRec> defs = h->defs_host;
-    std::vector<u64> instrs = h->instrs_host;
-    defs.push_back(r);
-    instrs.insert(instrs.end(), code.instr.begin(), code.instr.end());
-    std::swap(defs, h->defs_host);
-    std::swap(instrs, h->instrs_host);
-    upload_book(h);
+    std::vector<DefRec> defs{r};
+    validate_book(defs, code.instr);
+    const hvm64::DeviceBook b = hvm64::build_device_book(defs, code.instr);
+    drop_plan(h);
+    ensure_trg(h, b.max_slots);
+    const u64 dw = sizeof(DefRec) / 8, words = dw + 1 + b.instrs.size() + b.tmpl.size();
+    if (words > h->d_net_cap) {
+      dfree(h->d_net);
+      h->d_net_cap = 0;
+      hip_check(hipMalloc(&h->d_net, 2 * words * sizeof(u64)), "hipMalloc net code");
+      h->d_net_cap = 2 * words;
+    }
+    std::vector<u64> w(words);
+    std::memcpy(w.data(), defs.data(), sizeof(DefRec));
+    w[dw] = b.cdefs[0];
+    std::copy(b.instrs.begin(), b.instrs.end(), w.begin() + dw + 1);
+    std::copy(b.tmpl.begin(), b.tmpl.end(), w.begin() + dw + 1 + b.instrs.size());
+    hip_check(hipMemcpy(h->d_net, w.data(), words * sizeof(u64), hipMemcpyHostToDevice), "upload net code");
     Params P = make_params(h, ~0ull);
-    hip_check(launch_exec(P, (u32)h->defs_host.size() - 1, mkport(T_VAR, 0, h->root_cell), 0, h->stream),
-              "launch encode");
-    sync_globals(h);
-    std::swap(defs, h->defs_host);
-    std::swap(instrs, h->instrs_host);
-    upload_book(h);
+    P.defs = (const DefRec *)h->d_net;
+    P.cdefs = h->d_net + dw;
+    P.instrs = h->d_net + dw + 1;
+    P.tmpl = P.instrs + b.instrs.size();
+    hip_check(launch_exec(P, 0, mkport(T_VAR, 0, h->root_cell), 0, h->stream), "launch encode");
+    sync_globals(h, true);
   });
 }
 
 int hvm_gpu_normal(hvm_gpu *h) {
   return guarded(h, [&] {
     Params P = make_params(h, ~0ull);
+    // (an error of the expansion ends the reduction at its first look)
     hip_check(launch_expand(P, h->root_cell, h->stream), "launch expand");
-    sync_globals(h);
-    h->root_cell = h->last.result;
-    run_reduce(h, ~0ull);
+    try {
+      run_reduce(h, ~0ull, false, true);
+    } catch (Error &) {
+      h->root_cell = h->last.root;
+      throw;
+    }
+    h->root_cell = h->last.root;
   });
 }
 

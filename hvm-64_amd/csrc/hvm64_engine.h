@@ -121,9 +121,10 @@ struct alignas(128) Globals {
   u64 _p4[15];
   u32 err;         // first error code
   u32 err_info;
-  u64 result;      // kernel-specific result word (new root cell, readback length)
+  u64 result;      // kernel-specific result word (readback length, an error's address)
   u64 captured_n;  // redexes recorded by calls on inert definitions
-  u64 _p5[13];
+  u64 root;        // the new root cell of the last expand
+  u64 _p5[12];
   u64 rw[RW_SLOTS];  // cumulative counters (RW_POPS: redexes popped)
   u64 _p6[16 - RW_SLOTS];
   u64 st[ST_SLOTS];  // scheduler statistics of the last reduce launch
@@ -147,6 +148,9 @@ struct Params {
   u64 *queue;          // global redex ring, 2 words per slot
   u64 qmask;           // ring slots - 1
   Globals *g;
+  u64 *g_host;         // pinned host memory: a copy of *g, written by kernels that end a host call
+  u64 *rb_host;        // pinned host memory: readback results of up to rb_host_cap words
+  u64 rb_host_cap;
   u32 ndefs;
   u32 trg_slots;       // registers per lane
   u32 total_waves;     // waves in the reduce grid

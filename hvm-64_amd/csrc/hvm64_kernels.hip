@@ -47,23 +47,67 @@ __global__ void k_fill(u64 *words, u64 n, u64 value) {
   for (; i < n; i += stride) words[i] = value;
 }
 
+// Copies the control block to the host's view of it (pinned memory), so that
+// reading it after a launch costs the host no copy of its own: a blocking copy
+// of 1.5 KiB is 10-15 us, the whole boot of a small net 35.  One wave.
+DEV void mirror_globals(const Params &P, u32 lane) {
+  const u64 *gw = (const u64 *)P.g;
+  for (u32 i = lane; i < sizeof(Globals) / 8; i += 64) HVM_ST_SYS(P.g_host + i, gld((u64 *)gw + i));
+}
+__global__ void k_mirror(Params P) { mirror_globals(P, threadIdx.x); }
+
+// Net::new: every allocation ring, the control block, the idle set and the
+// mailboxes as they are at the start, the root var cell empty, and the global
+// redex ring's slots [q0, q1) (those that may hold a redex; a finished
+// reduction has consumed them all) empty.
+__global__ void k_reset(Params P, u64 q0, u64 q1) {
+  const u64 tid = (u64)blockIdx.x * blockDim.x + threadIdx.x, stride = (u64)gridDim.x * blockDim.x;
+  for (u64 i = q0 + tid; i < q1; i += stride) {
+    u64 *slot = P.queue + (i & P.qmask) * 2;
+    slot[0] = 0;
+    slot[1] = 0;
+  }
+  u64 *gw = (u64 *)P.g;
+  for (u64 i = tid; i < sizeof(Globals) / 8; i += stride) gw[i] = 0;
+  for (u64 i = tid; i < (u64)P.total_waves * 64; i += stride) P.alloc_pos[i] = 0;
+  for (u64 i = tid; i < P.idle_words; i += stride) P.idle_bits[i] = 0;
+  for (u64 i = tid; i < (u64)P.total_waves * MBOX_WORDS; i += stride) P.mbox[i] = 0;
+  if (tid == 0) P.heap[ROOT0_WORD] = P_NONE;
+}
+
+// What a reduction finds at its start: no budget spent, no statistics, no idle
+// waves, empty mailboxes.
+DEV void prepare_reduce(const Params &P, u64 tid, u64 stride) {
+  for (u64 i = tid; i < ST_SLOTS; i += stride) P.g->st[i] = 0;
+  for (u64 i = tid; i < P.idle_words; i += stride) P.idle_bits[i] = 0;
+  for (u64 i = tid; i < (u64)P.total_waves * MBOX_WORDS; i += stride) P.mbox[i] = 0;
+  if (tid == 0) P.g->done = 0;
+}
+__global__ void k_prepare(Params P) {
+  prepare_reduce(P, (u64)blockIdx.x * blockDim.x + threadIdx.x, (u64)gridDim.x * blockDim.x);
+}
+
 // Run one definition's instructions with t0 = `t0` on lane 0 of wave 0:
 // Net::boot (net.rs:30-32, counts one dref) or Host::encode_net
-// (encode.rs:31-35, counts nothing).  Redexes go to the global ring.
+// (encode.rs:31-35, counts nothing).  Redexes go to the global ring.  The
+// wave's other lanes only help to copy the control block to the host.
 __global__ void k_exec(Params P, u32 def, u64 t0, u32 count_dref) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
   __shared__ pair s_pl[LINK_CAP * 64];
   __shared__ u64 s_t[LDS_SLOTS * 64];
-  Lane L;
-  lane_init(L, P, 0, 0);
-  L.PL = s_pl;
-  L.T_lds = s_t;
-  if (count_dref) L.rw[RW_DREF]++;
-  run_def(L, def, t0);
-  publish();
-  lane_finish(L);
-  for (u32 k = 0; k < RW_SLOTS; k++)
-    if (L.rw[k]) __hip_atomic_fetch_add(&P.g->rw[k], (u64)L.rw[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) {
+    Lane L;
+    lane_init(L, P, 0, 0);
+    L.PL = s_pl;
+    L.T_lds = s_t;
+    if (count_dref) L.rw[RW_DREF]++;
+    run_def(L, def, t0);
+    publish();
+    lane_finish(L);
+    for (u32 k = 0; k < RW_SLOTS; k++)
+      if (L.rw[k]) __hip_atomic_fetch_add(&P.g->rw[k], (u64)L.rw[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    publish();
+  }
+  mirror_globals(P, threadIdx.x);
 }
 
 // A batch of independent nets: net i gets a fresh root cell (roots[i]) and
@@ -154,9 +198,13 @@ __global__ void k_root_ports(Params P, u32 n, const u64 *roots, u64 *out) {
 
 // Net::expand (net.rs:65-69): a fresh root cell R2 and an ExpandDef whose
 // `out` is R2's other endpoint, linked to the old root.  Writes R2's address
-// to g->result.
+// to g->root.  The blocks after the first prepare the reduction that follows.
 __global__ void k_expand(Params P, u64 old_root_cell) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  if (blockIdx.x != 0) {
+    prepare_reduce(P, (u64)(blockIdx.x - 1) * blockDim.x + threadIdx.x, (u64)(gridDim.x - 1) * blockDim.x);
+    return;
+  }
+  if (threadIdx.x != 0) return;
   __shared__ pair s_pl[LINK_CAP * 64];
   Lane L;
   lane_init(L, P, 0, 0);
@@ -168,7 +216,7 @@ __global__ void k_expand(Params P, u64 old_root_cell) {
   flush_links(L, np);
   publish();
   lane_finish(L);
-  P.g->result = r2;
+  P.g->root = r2;
   for (u32 k = 0; k < RW_SLOTS; k++)
     if (L.rw[k]) __hip_atomic_fetch_add(&P.g->rw[k], (u64)L.rw[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -1091,6 +1139,8 @@ __global__ __launch_bounds__(RB_THREADS) void k_readback(Params P, u64 root_cell
       P.g->err = ERR_READBACK;
       P.g->result = 0;
     }
+    __syncthreads();
+    if (t < 64) mirror_globals(P, t);
     return;
   }
   for (u64 k = t; k < nroots; k += RB_THREADS) {
@@ -1153,6 +1203,8 @@ __global__ __launch_bounds__(RB_THREADS) void k_readback(Params P, u64 root_cell
       P.g->err = ERR_READBACK;
       P.g->result = 0;
     }
+    __syncthreads();
+    if (t < 64) mirror_globals(P, t);
     return;
   }
   if (t == 0) HVM_ST(&lev[L], a);  // a: every entry
@@ -1186,6 +1238,8 @@ __global__ __launch_bounds__(RB_THREADS) void k_readback(Params P, u64 root_cell
       P.g->err = ERR_READBACK;
       P.g->result = s_n;
     }
+    __syncthreads();
+    if (t < 64) mirror_globals(P, t);
     return;
   }
   for (u64 l = 0; l < L; l++) {
@@ -1202,7 +1256,12 @@ __global__ __launch_bounds__(RB_THREADS) void k_readback(Params P, u64 root_cell
     }
     __syncthreads();
   }
+  // a result of up to P.rb_host_cap words goes to the host's buffer as well
+  if (s_n <= P.rb_host_cap)
+    for (u64 i = t; i < s_n; i += RB_THREADS) HVM_ST_SYS(P.rb_host + i, HVM_LD(&out[i]));
   if (t == 0) P.g->result = s_n;
+  __syncthreads();
+  if (t < 64) mirror_globals(P, t);
 }
 
 // ---------------------------------------------------------------------------
@@ -1253,7 +1312,21 @@ hipError_t launch_exec(const Params &P, u32 def, u64 t0, u32 count_dref, hipStre
   return hipGetLastError();
 }
 hipError_t launch_expand(const Params &P, u64 old_root_cell, hipStream_t st) {
-  hipLaunchKernelGGL(k_expand, dim3(1), dim3(64), 0, st, P, old_root_cell);
+  hipLaunchKernelGGL(k_expand, dim3(1 + 64), dim3(64), 0, st, P, old_root_cell);
+  return hipGetLastError();
+}
+hipError_t launch_prepare(const Params &P, hipStream_t st) {
+  hipLaunchKernelGGL(k_prepare, dim3(64), dim3(256), 0, st, P);
+  return hipGetLastError();
+}
+hipError_t launch_mirror(const Params &P, hipStream_t st) {
+  hipLaunchKernelGGL(k_mirror, dim3(1), dim3(64), 0, st, P);
+  return hipGetLastError();
+}
+hipError_t launch_reset(const Params &P, u64 q0, u64 q1, hipStream_t st) {
+  const u64 n = q1 - q0 > (u64)P.total_waves * MBOX_WORDS ? q1 - q0 : (u64)P.total_waves * MBOX_WORDS;
+  const u64 blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(k_reset, dim3((u32)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, st, P, q0, q1);
   return hipGetLastError();
 }
 hipError_t launch_boot_batch(const Params &P, u32 n, const u32 *defs, u64 *roots, u32 max_blocks, hipStream_t st) {

@@ -722,6 +722,18 @@ DEV void redux(Lane &L, u64 a, u64 b) {
 // a longer run than MAX_CHAIN rounds means a corrupted net.
 static const u32 MAX_CHAIN = 1u << 24;
 
+// A lane on a long chain, every CHAIN_LOOK rounds: has the launch failed?
+// After an allocation failed the dump cell stands in for the missing node,
+// and lanes that meet there hand each other's ports round for as long as
+// MAX_CHAIN lets them, while what the lane recorded itself waits for the end
+// of its task (a planned batch that ran out of nodes took 30 to 90 s to
+// report it; it takes as long as the launch up to there).
+static const u32 CHAIN_LOOK = 256;
+DEV bool launch_failed(Lane &L) {
+  lane_report(L);
+  return HVM_LD(&L.P->g->err) != 0;
+}
+
 // Every producer checks the room it needs (interp_run: one link per
 // instruction; a rule: at most four, into an empty list).
 DEV void push_link(Lane &L, u32 &np, u64 a, u64 b) {
@@ -736,10 +748,12 @@ DEV void push_link(Lane &L, u32 &np, u64 a, u64 b) {
 // many passes as the lane with the most of them has.
 DEV void flush_links(Lane &L, u32 &np) {
   for (u32 round = 0; np > 0; round++) {
-    if (round > MAX_CHAIN) {
-      fail(L, ERR_BADPTR, BAD_CHAIN);
-      np = 0;
-      return;
+    if (round % CHAIN_LOOK == CHAIN_LOOK - 1) {
+      if (round > MAX_CHAIN) fail(L, ERR_BADPTR, BAD_CHAIN);
+      if (launch_failed(L)) {
+        np = 0;
+        return;
+      }
     }
     const u32 cnt = np < 4 ? np : 4;
     np -= cnt;
@@ -805,12 +819,12 @@ DEV u64 follow(Lane &L, u64 p, bool go) {
         go = is_endpoint(v);
       }
     }
-    if (hop >= MAX_CHAIN) {
-      if (go) {
-        fail(L, ERR_BADPTR, BAD_RESOLVE);
+    if (hop % CHAIN_LOOK == CHAIN_LOOK - 1 && go) {
+      if (hop >= MAX_CHAIN) fail(L, ERR_BADPTR, BAD_RESOLVE);
+      if (launch_failed(L)) {
         p = P_ERA;
+        go = false;
       }
-      break;
     }
   }
   return p;

@@ -158,3 +158,25 @@ def test_planned_batch_4096_against_oracle(oracle):
             assert plan.rwts.as_dict() == total
     finally:
         heap.close()
+
+
+def test_planned_batch_out_of_nodes_ends_soon():
+    """A batch whose nets need twice the heap reports it within seconds: lanes
+    without a node meet in one dump cell, and no chain through it goes on
+    after the launch has failed."""
+    import time
+    import hvm64
+    from hvm64 import configs
+    book, nets, table = configs.batch_mix(64, seed=14)
+    heap = hvm64.Heap(768 << 20)
+    try:
+        host = hvm64.Host(book, heap)
+        defs = [host.defs[table[v][0]] for v in nets]
+        plan = hvm64.PlannedBatch(heap, defs, hvm64.arena_sizes(heap, defs, margin=0.3, extra=0))
+        t = time.perf_counter()
+        with pytest.raises(hvm64.HvmError) as e:
+            plan.run()
+        assert e.value.kind == "OOM"
+        assert time.perf_counter() - t < 5
+    finally:
+        heap.close()

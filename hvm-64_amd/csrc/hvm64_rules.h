@@ -62,11 +62,14 @@ namespace hvm {
 #if defined(__HIPCC__) || defined(__HIP__)
 DEV u32 uniform(u32 v) { return __builtin_amdgcn_readfirstlane(v); }
 DEV u32 lane_at(u32 v, u32 i) { return __builtin_amdgcn_readlane(v, i); }
+DEV u32 lane_from(u32 v, u32 i) { return (u32)__builtin_amdgcn_ds_bpermute((int)(i * 4), (int)v); }  // each lane its own i
 #else
 DEV u32 uniform(u32 v) { return v; }
 DEV u32 lane_at(u32 v, u32) { return v; }
+DEV u32 lane_from(u32 v, u32) { return v; }
 #endif
 DEV u64 uniform(u64 v) { return (u64)uniform((u32)v) | (u64)uniform((u32)(v >> 32)) << 32; }
+DEV u64 lane_from(u64 v, u32 i) { return (u64)lane_from((u32)v, i) | (u64)lane_from((u32)(v >> 32), i) << 32; }
 DEV u64 lane_at(u64 v, u32 i) { return (u64)lane_at((u32)v, i) | (u64)lane_at((u32)(v >> 32), i) << 32; }
 
 static const u32 WAVES_PER_BLOCK = 4;
@@ -417,41 +420,47 @@ DEV u32 net_of_port(const Params &P, u64 p, u32 dflt) {
 // restart in between; with an atomic per lane the words of a few dozen slots
 // were the hottest lines of the launch.)  A slot's arena is SERVE_SUB
 // sub-arenas; the lane that adds goes through them in turn.
+// The lanes first find their slot's sum and their place in it, without a
+// memory access; then the first lane of every slot adds, all of them at once,
+// and the others take the result from it.  (Each slot's add waited for before
+// the next slot's turn: 128 requests on 32 slots 137 ms; this way 131 ms.)
 DEV void arena_room_serve(Lane &L, u32 need) {
   const Params &P = *L.P;
-  const u64 len = (u64)P.sub_granules << P.gran_shift;
+  u32 lead = 0, before = 0, sum = 0;
   for (u64 todo = HVM_BALLOT(true); todo;) {
-    const u32 lead = (u32)__builtin_ctzll(todo);
-    const u32 net = lane_at(L.cur_net, lead);
-    const bool mine = L.cur_net == net;
-    const u64 same = HVM_BALLOT(mine);
-    u32 sum = 0, before = 0;
+    const u32 first = (u32)__builtin_ctzll(todo);
+    const bool mine = L.cur_net == lane_at(L.cur_net, first);
+    u32 all = 0, below = 0;
     for (u32 b = 0; HVM_ANY(need >> b != 0); b++) {
       const u64 m = HVM_BALLOT(mine && ((need >> b) & 1));
-      sum += (u32)__builtin_popcountll(m) << b;
-      before += HVM_BELOW(m) << b;
+      all += (u32)__builtin_popcountll(m) << b;
+      below += HVM_BELOW(m) << b;
     }
-    // (a full sub-arena gives its add back and the next one is tried)
-    const u32 first = lane_at(L.rw[RW_POPS], lead) + lead;
-    u64 w = 0;
-    bool fits = false;
-    for (u32 k = 0; k < SERVE_SUB && !fits; k++) {
-      u64 *const word = &P.arena_word[net * SERVE_SUB + ((first + k) & (SERVE_SUB - 1))];
-      if (L.lane_id == lead) w = HVM_FAA(word, (u64)sum);
-      w = lane_at(w, lead);
-      fits = (w & 0xFFFFFFFFull) + sum <= len;
-      if (!fits && L.lane_id == lead) HVM_FAA(word, (u64)0 - sum);
-    }
-    if (mine) {
-      L.a_pos = ((w >> 32) << P.gran_shift) + (w & 0xFFFFFFFFull) + before;
-      L.a_end = L.a_pos + need;
-      if (!fits) {
-        fail(L, ERR_OOM, OOM_POOL);
-        L.a_end = L.a_pos;
-      }
-    }
-    todo &= ~same;
+    lead = mine ? first : lead;
+    sum = mine ? all : sum;
+    before = mine ? below : before;
+    todo &= ~HVM_BALLOT(mine);
   }
+  u64 w = 0;
+  bool fits = false;
+  if (L.lane_id == lead) {
+    const u64 len = (u64)P.sub_granules << P.gran_shift;
+    u64 *const words = &P.arena_word[(u64)L.cur_net * SERVE_SUB];
+    // (a full sub-arena gives its add back and the next one is tried)
+    const u32 k0 = L.rw[RW_POPS] + lead;
+    for (u32 k = 0; k < SERVE_SUB && !fits; k++) {
+      u64 *const word = &words[(k0 + k) & (SERVE_SUB - 1)];
+      w = HVM_FAA(word, (u64)sum);
+      fits = (w & 0xFFFFFFFFull) + sum <= len;
+      if (!fits) HVM_FAA(word, (u64)0 - sum);
+    }
+    w = fits ? ((w >> 32) << P.gran_shift) + (w & 0xFFFFFFFFull) : ~0ull;
+  }
+  w = lane_from(w, lead);
+  fits = w != ~0ull;
+  L.a_pos = fits ? w + before : 0;
+  L.a_end = fits ? L.a_pos + need : 0;
+  if (!fits) fail(L, ERR_OOM, OOM_POOL);
 }
 
 // Makes room for `need` consecutive nodes of the running task's net.  Right
@@ -1416,7 +1425,7 @@ DEV void serve_complete(Lane &L, u32 s) {
 // One atomic per slot and wave: the changes of the lanes on a slot are summed,
 // and the first of those lanes sends the sum and looks at it later (an atomic
 // per lane, all slots' words on a few lines, held every iteration up: 128
-// requests on 32 slots, 350 ms; with this and arena_room_serve 136 ms).  All lanes call it; `ran`: the lane ran a
+// requests on 32 slots, 350 ms; with this and arena_room_serve 131 ms).  All lanes call it; `ran`: the lane ran a
 // task or a boot.
 DEV void serve_account_deferred(Lane &L, bool ran) {
   L.acct_delta = 0;

@@ -133,8 +133,12 @@ const u32 NO_NET_HOST = 0xFFFFFFFFu;
 // First word of a book image written by hvm_book_encode: "HVM64BK1".
 const u64 BOOK_IMAGE_MAGIC = 0x314B4234364D5648ull;
 
+// (the error is taken off HIP's record as well: the next launch's check reads
+// that record, and an allocation that failed for one handle is not its error)
 void hip_check(hipError_t e, const char *what) {
-  if (e != hipSuccess) throw Error(HVM_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();
+  throw Error(HVM_E_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
 template <class T>

@@ -240,11 +240,13 @@ class DefRef:
 
 
 class _Defs:
-    def __init__(self, host):
-        self._host = host
+    def __init__(self, heap):
+        # the heap, not the Host: no reference cycle keeps a dropped heap's
+        # device memory until the next garbage collection
+        self._heap = heap
 
     def __getitem__(self, name):
-        h = self._host.heap
+        h = self._heap
         i = ctypes.c_uint32()
         h._check(h._lib.hvm_gpu_def_id(h._h, name.encode(), ctypes.byref(i)))
         return DefRef(name, i.value)
@@ -328,7 +330,7 @@ class Host:
             del keep
         else:
             raise ValueError(via)
-        self.defs = _Defs(self)
+        self.defs = _Defs(heap)
 
     def readback(self, net):
         """Host::readback + Display (host/src/readback.rs:23-33): normal form text."""

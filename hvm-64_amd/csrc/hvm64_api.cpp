@@ -187,8 +187,15 @@ Params make_params(hvm_gpu *h, u64 limit) {
   P.mbox = h->mbox;
   P.idle_words = h->idle_words;
   P.t_lds = h->max_nslots <= reduce_lds_slots() ? 1 : 0;
-  P.book_lds =
-      (u64)h->ndefs * 5 + P.instr_words + P.lab_words + P.tmpl_words <= reduce_book_lds_words() ? 1 : 0;
+  // What of the book goes to LDS: all of it; or all but the instructions; or
+  // nothing.  A call reads several words of its records, label bits and
+  // template, each on its own, and a redex's ring is found in the record (by
+  // length; without the record, by index); of the instructions two words are
+  // read at a time, once, in order, so they are what is left out.  A book of
+  // 394 definitions, 16,340 words (4,922 without the instructions), 96 nets:
+  // 80.9 ms with nothing in LDS, 77.9 ms with the rest there.
+  const u64 rest = (u64)h->ndefs * 5 + P.lab_words + P.tmpl_words, room = reduce_book_lds_words();
+  P.book_lds = rest + P.instr_words <= room ? BOOK_ALL : rest <= room ? BOOK_REST : BOOK_GLOBAL;
   P.limit = limit;
   P.timeout_ticks = h->timeout_ticks;
   return P;

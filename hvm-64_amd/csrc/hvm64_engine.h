@@ -130,6 +130,10 @@ struct alignas(128) Globals {
   u64 st[ST_SLOTS];  // scheduler statistics of the last reduce launch
 };
 
+// What of the book a reduce launch keeps in LDS: nothing, all but the
+// instructions, or all of it.
+enum BookLds : u32 { BOOK_GLOBAL = 0, BOOK_REST = 1, BOOK_ALL = 2 };
+
 // Launch-time parameters of every kernel.
 struct Params {
   u64 *heap;           // heap[(addr - HVM_HEAP_OFF) >> 3] is the word at engine address `addr`
@@ -154,7 +158,7 @@ struct Params {
   u32 ndefs;
   u32 trg_slots;       // registers per lane
   u32 total_waves;     // waves in the reduce grid
-  u32 book_lds;        // 1: the reduce kernel copies the book into LDS
+  u32 book_lds;        // what of the book the reduce kernel copies into LDS (BookLds)
   u32 instr_words;     // words in `instrs`
   u32 lab_words;       // words in `labbits`
   u32 t_lds;           // 1: every definition's trg registers fit in LDS

@@ -477,13 +477,15 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   __shared__ u32 s_act, s_idle, s_given[WAVES_PER_BLOCK];
   const u32 wib = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // the book, copied into LDS when it fits (the host decides: P.book_lds)
+  // (BOOK_REST: all but its instructions)
   const u32 nd = P.ndefs * 4;
-  const u32 b_cdef = nd + P.instr_words + P.lab_words, b_tmpl = b_cdef + P.ndefs;
+  const u32 ins_words = LDS || P.book_lds == BOOK_ALL ? P.instr_words : 0;
+  const u32 b_lab = nd + ins_words, b_cdef = b_lab + P.lab_words, b_tmpl = b_cdef + P.ndefs;
   if (LDS || P.book_lds) {
     const u64 *defs = (const u64 *)P.defs;
     for (u32 i = threadIdx.x; i < nd; i += blockDim.x) s_book[i] = defs[i];
-    for (u32 i = threadIdx.x; i < P.instr_words; i += blockDim.x) s_book[nd + i] = P.instrs[i];
-    for (u32 i = threadIdx.x; i < P.lab_words; i += blockDim.x) s_book[nd + P.instr_words + i] = P.labbits[i];
+    for (u32 i = threadIdx.x; i < ins_words; i += blockDim.x) s_book[nd + i] = P.instrs[i];
+    for (u32 i = threadIdx.x; i < P.lab_words; i += blockDim.x) s_book[b_lab + i] = P.labbits[i];
     for (u32 i = threadIdx.x; i < P.ndefs; i += blockDim.x) s_book[b_cdef + i] = P.cdefs[i];
     for (u32 i = threadIdx.x; i < P.tmpl_words; i += blockDim.x) s_book[b_tmpl + i] = P.tmpl[i];
   }
@@ -513,8 +515,8 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
   L.FC = &s_cache[ARENAS ? 0 : wib][ARENAS ? 0 : lane];
   if (LDS || P.book_lds) {
     L.book = HVM_TO_LDS(s_book);
-    L.book_ins = nd;
-    L.book_lab = nd + P.instr_words;
+    L.book_ins = LDS || P.book_lds == BOOK_ALL ? nd : NO_INS;
+    L.book_lab = b_lab;
     L.book_cdef = b_cdef;
     L.book_tmpl = b_tmpl;
   }
@@ -1357,7 +1359,7 @@ hipError_t launch_root_ports(const Params &P, u32 n, const u64 *roots, u64 *out,
 hipError_t launch_reduce(const Params &P, u32 blocks, hipStream_t st) {
   const dim3 grid(blocks), block(WAVES_PER_BLOCK * 64);
   // the LDS instantiation when the book and every trg register fit there
-  const bool lds = P.book_lds && P.t_lds;
+  const bool lds = P.book_lds == BOOK_ALL && P.t_lds;
 #define HVM_REDUCE(A, S, T)                                                     \
   do {                                                                          \
     if (lds) hipLaunchKernelGGL((k_reduce<A, S, T, true>), grid, block, 0, st, P); \

@@ -88,7 +88,9 @@ DEV u32 ring_stat(u32 c) { return c == CLS_OTHER ? 3u : c >= CLS_CALL ? 2u : c; 
 static const u32 LDS_SLOTS = 10;   // trg registers per lane kept in LDS
 static const u32 LINK_CAP = 6;     // deferred links per lane (LDS)
 // A book of at most BOOK_LDS_WORDS words (definition records, instructions,
-// label bits) is copied into every block's LDS by the reduce kernel.
+// label bits, compiled-definition records, templates) is copied into every
+// block's LDS by the reduce kernel; of a larger one all but the instructions,
+// when that fits.
 static const u32 BOOK_LDS_WORDS = 6144;
 
 // ---------------------------------------------------------------------------
@@ -211,9 +213,9 @@ struct Lane {
   u32 *bag_top;
   const u32 *bag_bot;
   // the book in LDS (nullptr: read it from global memory): definition
-  // records at 0 (4 words each), instructions at book_ins, label bits at
-  // book_lab, compiled-definition records at book_cdef, templates at
-  // book_tmpl
+  // records at 0 (4 words each), instructions at book_ins (NO_INS: they are
+  // read from global memory), label bits at book_lab, compiled-definition
+  // records at book_cdef, templates at book_tmpl
   lds_u64 *book;
   u32 book_ins, book_lab, book_cdef, book_tmpl;
   // counters
@@ -256,6 +258,9 @@ DEV void lane_report(Lane &L) {
 
 // The book is read from LDS (L.book) rather than from global memory.
 DEV bool has_book(const Lane &L) { return L.lds_all || L.book != nullptr; }
+static const u32 NO_INS = 0xFFFFFFFFu;
+// Its instructions too.
+DEV bool has_ins(const Lane &L) { return L.lds_all || (L.book != nullptr && L.book_ins != NO_INS); }
 
 DEV u64 dump_addr() { return HVM_HEAP_OFF + DUMP_WORD * 8; }
 
@@ -1220,7 +1225,7 @@ DEV void interp_begin(Lane &L, Interp &I, const DefRec &d, u64 t0, u64 cdef) {
 
 // The next instruction's two words.
 DEV void fetch(const Lane &L, const Interp &I, u64 &w0, u64 &w1) {
-  if (has_book(L)) {
+  if (has_ins(L)) {
     w0 = L.book[L.book_ins + I.ipw];
     w1 = L.book[L.book_ins + I.ipw + 1];
   } else {

@@ -299,8 +299,6 @@ DEV u32 row0_max(u32 v) {
   return lane_at(v, 15);
 }
 
-// Moves `cnt` redexes, the oldest of class `c`, from the wave's rings to the
-// global ring (all lanes; lane 0 updates the counters).  Returns S after.
 // Takes the next k (<= 64) redexes of the global ring, whose count in S this
 // wave has already claimed, into its rings (the caller checks they fit).
 DEV void claim_global(const Params &P, Lane &L, pair *bag, u32 *top_c, u32 k, u32 lane, u64 t_end) {
@@ -355,6 +353,8 @@ DEV void take_mail(u64 *box, Lane &L, pair *bag, u32 *top_c, u32 k, u32 lane, u6
   __builtin_amdgcn_wave_barrier();
 }
 
+// Moves `cnt` redexes, the oldest of class `c`, from the wave's rings to the
+// global ring (all lanes; lane 0 updates the counters).  Returns S after.
 DEV u64 spill_to_global(const Params &P, const pair *bag, u32 *bot_c, u32 c, u32 cnt, u32 lane, u32 bot, u32 &err) {
   // the nodes these redexes reach must be in memory before a claimer can
   // read the ring slots (which it may do before S counts them)

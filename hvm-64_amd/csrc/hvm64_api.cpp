@@ -208,6 +208,7 @@ void sync_globals(hvm_gpu *h, bool mirrored = false) {
   hip_check(hipStreamSynchronize(h->stream), "kernel");
   std::memcpy(&h->last, h->pin, sizeof(Globals));
   if (h->last.err) {
+    h->ring_unknown = true;
     u32 e = h->last.err;
     int code = e == ERR_OOM ? HVM_E_OOM
                : e == ERR_UNIMPL ? HVM_E_UNIMPL_PAIR
@@ -291,18 +292,13 @@ void upload_book(hvm_gpu *h) {
   ensure_trg(h, b.max_slots);
 }
 
-// Net::new.  The heap is filled with FREE once, when the handle opens; a
-// reset rewinds every allocation ring instead.  That is enough for a fresh
-// net: a ring's first lap overwrites its slots without reading them, and
-// later laps only reuse slots whose words read FREE, so words left by a
-// previous net are either overwritten or skipped, never read as live.
 // The control block, the rings, the idle set and the mailboxes.  The global
 // redex ring (1 GiB) is cleared where it may hold redexes: every redex taken
 // from it leaves zeros, so after a reduction that ended well that is
 // [q_head, q_tail), usually nothing; after an error, all of it.  (Clearing it
 // all took 170 us of every Net::new, a quarter of a small program's run.)
 void clear_state(hvm_gpu *h) {
-  const bool all = h->ring_unknown || h->last.err != 0 || h->last.q_tail - h->last.q_head > h->qslots;
+  const bool all = h->ring_unknown || h->last.q_tail - h->last.q_head > h->qslots;
   hip_check(launch_reset(make_params(h, ~0ull), all ? 0 : h->last.q_head, all ? h->qslots : h->last.q_tail, h->stream),
             "reset");
   hip_check(hipStreamSynchronize(h->stream), "reset");
@@ -310,6 +306,11 @@ void clear_state(hvm_gpu *h) {
   h->ring_unknown = false;
 }
 
+// Net::new.  The heap is filled with FREE once, when the handle opens; a
+// reset rewinds every allocation ring instead.  That is enough for a fresh
+// net: a ring's first lap overwrites its slots without reading them, and
+// later laps only reuse slots whose words read FREE, so words left by a
+// previous net are either overwritten or skipped, never read as live.
 void reset_net(hvm_gpu *h, bool fill) {
   fill = fill || h->heap_dirty;
   h->heap_dirty = false;
@@ -628,18 +629,14 @@ void replan(hvm_gpu *h, const hvm_batch_tuning t) {  // a copy: make_plan clears
 void run_plan(hvm_gpu *h) {
   hvm_gpu::Plan &p = h->plan;
   if (!p.n) throw Error(HVM_E_ARG, "no batch planned");
+  // (the batch's reset kernel rewinds the redex ring but clears no slot: what
+  // an unfinished or failed reduction left there is cleared here)
+  if (h->ring_unknown || h->last.q_head != h->last.q_tail) clear_state(h);
   hip_check(hipEventRecord(h->ev0, h->stream), "event");
   if (p.exec) hip_check(hipGraphLaunch(p.exec, h->stream), "graph launch");
   else plan_steps(h);
   hip_check(hipEventRecord(h->ev1, h->stream), "event");
-  try {
-    sync_globals(h);
-  } catch (Error &) {
-    // a failed reduction may leave redexes in the global ring
-    (void)launch_fill(h->queue, h->qslots * 2, 0, h->stream);
-    (void)hipStreamSynchronize(h->stream);
-    throw;
-  }
+  sync_globals(h);
   float ms = 0;
   hip_check(hipEventElapsedTime(&ms, h->ev0, h->ev1), "elapsed");
   h->last_ms = ms;

@@ -237,8 +237,8 @@ __global__ void k_expand(Params P, u64 old_root_cell) {
 // idle wave elsewhere, through its mailbox.  With more blocks active the
 // atomics on S and the idle set cost more than the passes they save (bitonic
 // 2^16: 113 ms; sharing beyond the block without that bound 220 ms), and a
-// batch whose global ring is stocked does not share at all: there fuller
-// passes count.  Measured without and with: Church c2^c9 4.50 -> 3.45 ms,
+// batch whose global ring is stocked, or with more blocks active, does not
+// share at all: there fuller passes count.  Measured without and with: Church c2^c9 4.50 -> 3.45 ms,
 // bitonic 2^6 7.08 -> 5.67 ms, 2^11 32.2 -> 28.4 ms, tree-sum 10 1.02 -> 0.84
 // ms; 2^16 109 -> 112 ms (shorter but more passes).
 //
@@ -847,12 +847,14 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     const u32 nth = (lane - rot) & 63;  // this lane runs the nth-newest redex
     u32 slot = ring_base(c) + ((top - 1 - nth) & (ring_cap(c) - 1)), total = take;
     if (lane == c) my_top -= take;
-    if (P.fill && c >= CLS_CALL && !limited && !admitting) {
-      // batched nets: the free lanes run redexes of the other call rings.
-      // Fewer, longer passes: where there is work for every lane that is
-      // throughput (512 nets 197 -> 181 ms); a single net waits for its
-      // longest definition more often (bitonic 2^6 7.5 -> 9.8 ms), so there a
-      // pass keeps to one ring
+    if (P.fill && (S_cache >> 32) > 0 && c >= CLS_CALL && !limited && !admitting) {
+      // batched nets, while the global ring holds work: the free lanes run
+      // redexes of the other call rings.  Fewer, longer passes: where there is
+      // work for every lane that is throughput (512 planned nets 197 -> 181
+      // ms); where there is not, a net waits for its longest definition more
+      // often (bitonic 2^6 alone 7.5 -> 9.8 ms; merging also while the ring is
+      // empty: 12 unplanned nets 56 ms instead of 49, 128 served ones 130
+      // instead of 113)
 #pragma unroll
       for (u32 q = CLS_CALL; q < NCLS; q++) {
         const u32 nq = q == c ? 0 : lane_at(my_n, q), tq = nq < 64 - total ? nq : 64 - total;
@@ -934,9 +936,11 @@ __global__ __launch_bounds__(WAVES_PER_BLOCK * 64) void k_reduce(Params P) {
     }
     // ---- idle waves of this block: each gets a whole ring, while this wave
     // has another one for its next pass
-    // (batched nets, while the global ring holds work: fuller iterations are
-    // worth more than busier waves)
-    const bool share_ok = !(P.fill && (S_cache >> 32) > 0);
+    // (batched nets, while the global ring holds work or many blocks are
+    // active: fuller iterations are worth more than busier waves.  100 planned
+    // nets: sharing whenever the ring is empty 110 ms, up to 128 blocks 98, up
+    // to 64 95)
+    const bool share_ok = !(P.fill && ((S_cache >> 32) > 0 || (u32)S_cache > SHARE_BLOCKS));
     u32 rings = 0;  // those with redexes, but for the one to run next
     if (share_ok) {
       key = row0_max(lane < NCLS ? ring_key(lane, my_n) : 0);

@@ -1354,6 +1354,9 @@ int hvm_gpu_encode_net_text(hvm_gpu *h, const char *net_text) {
     std::copy(b.tmpl.begin(), b.tmpl.end(), w.begin() + dw + 1 + b.instrs.size());
     hip_check(hipMemcpy(h->d_net, w.data(), words * sizeof(u64), hipMemcpyHostToDevice), "upload net code");
     Params P = make_params(h, ~0ull);
+    // where the registers are: by the net's own program, which may be wider
+    // than the book
+    P.t_lds = b.max_slots <= reduce_lds_slots() ? 1 : 0;
     P.defs = (const DefRec *)h->d_net;
     P.cdefs = h->d_net + dw;
     P.instrs = h->d_net + dw + 1;

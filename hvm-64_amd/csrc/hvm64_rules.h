@@ -1213,7 +1213,8 @@ DEV void interp_begin(Lane &L, Interp &I, const DefRec &d, u64 t0, u64 cdef) {
   }
   I.ipw = ioff * 2;
   I.left = ilen;
-  if (nslots > P.trg_slots) {  // the trg area is sized for the book
+  // the trg area is sized for the book, and is in LDS only for books that fit
+  if (nslots > (I.t_lds ? LDS_SLOTS : P.trg_slots)) {
     fail(L, ERR_BADPTR, BAD_SLOTS);
     I.left = 0;
     return;

@@ -105,7 +105,7 @@ struct hvm_gpu {
   struct Serve {
     bool running = false;
     u32 slots = 0;
-    u64 *dev = nullptr;        // pending | slot_root | slot_tag | free_ring | ctl | words | base0 | len | gmap | inl
+    u64 *dev = nullptr;        // pending | slot_root | slot_tag | free_ring | ctl | sub-arenas | gmap | inl
     u64 *host = nullptr;       // pinned: host_ctl | requests | completions
     u64 *host_dev = nullptr;   // its device address
     u64 req_cap = 0, done_cap = 0;
@@ -762,12 +762,11 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     sv.slots = slots;
     sv.req_cap = rq;
     sv.done_cap = dq;
-    // device: pending | root | tag | free ring | counters | words | base0 | len | gmap | inl
+    // device: pending | root | tag | free ring | counters | sub-arenas | gmap | inl
     const u64 inl_words = (u64)h->waves * 64 * SERVE_INL * 2;
-    const u64 nsub = (u64)slots * SERVE_SUB;
+    const u64 sub_words = (u64)slots * SERVE_WORDS;
     const u64 pending_words = (u64)slots * PENDING_STRIDE / 2;
-    const u64 words = pending_words + 3 * (u64)slots + SV_WORDS + 2 * nsub + (nsub + 1) / 2 + (gmap_len + 1) / 2 +
-                      inl_words + 64;
+    const u64 words = pending_words + 3 * (u64)slots + SV_WORDS + sub_words + (gmap_len + 1) / 2 + inl_words;
     hip_check(hipMalloc(&sv.dev, words * 8), "hipMalloc serving");
     u64 *w = sv.dev;
     u32 *pending = (u32 *)w;
@@ -780,25 +779,15 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     w += slots;
     u64 *ctl = w;
     w += SV_WORDS;
-    u64 *word = w;
-    w += nsub;
-    u64 *base0 = w;
-    w += nsub;
-    u32 *len = (u32 *)w;
-    w += (nsub + 1) / 2;
+    u64 *sub = w;
+    w += sub_words;
     u32 *gmap = (u32 *)w;
     w += (gmap_len + 1) / 2;
     u64 *inl = w;
-    w += inl_words;
-    u64 *nopool = w;  // the serving arenas do not grow: a pool and an overflow region of 0
-    std::vector<u64> h_word(nsub), h_base0(nsub), h_free(slots), h_ctl(SV_WORDS, 0);
-    std::vector<u32> h_len(nsub, (u32)sub_g), h_gmap(gmap_len, NO_NET_HOST);
+    std::vector<u64> h_free(slots), h_ctl(SV_WORDS, 0);
+    std::vector<u32> h_gmap(gmap_len, NO_NET_HOST);
     for (u32 i = 0; i < slots; i++) {
       const u64 b = first + (u64)i * slot_g;
-      for (u32 k = 0; k < SERVE_SUB; k++) {
-        h_base0[(u64)i * SERVE_SUB + k] = b + k * sub_g;
-        h_word[(u64)i * SERVE_SUB + k] = (b + k * sub_g) << 32;
-      }
       h_free[i] = (u64)i + 1;
       for (u64 g = b; g < b + slot_g; g++) h_gmap[g] = i;
     }
@@ -807,11 +796,8 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     hip_check(hipMemset(pending, 0, pending_words * 8), "init serving");
     hip_check(hipMemcpy(free_ring, h_free.data(), (size_t)slots * 8, hipMemcpyHostToDevice), "init serving");
     hip_check(hipMemcpy(ctl, h_ctl.data(), SV_WORDS * 8, hipMemcpyHostToDevice), "init serving");
-    hip_check(hipMemcpy(word, h_word.data(), nsub * 8, hipMemcpyHostToDevice), "init serving");
-    hip_check(hipMemcpy(base0, h_base0.data(), nsub * 8, hipMemcpyHostToDevice), "init serving");
-    hip_check(hipMemcpy(len, h_len.data(), nsub * 4, hipMemcpyHostToDevice), "init serving");
+    hip_check(hipMemset(sub, 0, sub_words * 8), "init serving");
     hip_check(hipMemcpy(gmap, h_gmap.data(), gmap_len * 4, hipMemcpyHostToDevice), "init serving");
-    hip_check(hipMemset(nopool, 0, 64 * 8), "init serving");
     // pinned host memory: control words | requests | completions
     const u64 hwords = SH_WORDS + 2 * rq + 4 * dq;
     hip_check(hipHostMalloc((void **)&sv.host, hwords * 8, hipHostMallocMapped | hipHostMallocCoherent),
@@ -829,20 +815,13 @@ int hvm_gpu_serve_start(hvm_gpu *h, uint32_t slots, uint64_t slot_nodes, uint64_
     P.gmap = gmap;
     P.gmap_len = gmap_len;
     P.gran_shift = gs;
-    P.arena_word = word;
-    P.arena_base0 = base0;
-    P.arena_len = len;
-    P.pool_next = nopool;
-    P.pool_end = 0;
-    P.ov_next = nopool + 16;
-    P.ov_end = 0;
+    P.arena_word = sub;
     P.n_nets = slots;
-    P.refill_granules = 1;
-    P.arena_chunk = 32;
     P.serve = 1;
     P.serve_slots = slots;
     P.pending = pending;
     P.sub_granules = (u32)sub_g;
+    P.serve_first = (u32)first;
     P.slot_root = slot_root;
     P.slot_tag = slot_tag;
     P.free_ring = free_ring;

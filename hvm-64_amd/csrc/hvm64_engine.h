@@ -204,7 +204,8 @@ struct Params {
   u32 serve;
   u32 serve_slots;
   u32 *pending;        // slot s: word s * PENDING_STRIDE
-  u32 sub_granules;    // granules of a slot's sub-arena
+  u32 sub_granules;    // granules of a slot's sub-arena (arena_word: SERVE_WORDS words a slot)
+  u32 serve_first;     // first granule of slot 0's arena; the others follow
   u64 *slot_root;      // root cell of each slot's net
   u64 *slot_tag;       // the request's tag
   u64 *free_ring;      // slot + 1 entries (0: not yet written), serve_slots entries
@@ -231,6 +232,7 @@ static const u32 SERVE_INL = 32;
 // A serving slot's arena is this many sub-arenas (consecutive, whole
 // granules each).
 static const u32 SERVE_SUB = 8;
+static const u32 SERVE_WORDS = 2 * SERVE_SUB;
 // The slots' counts of pending redexes stand on 128-byte lines of their own:
 // every task of a slot changes its count.
 static const u32 PENDING_STRIDE = 32;

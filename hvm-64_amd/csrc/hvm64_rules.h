@@ -419,12 +419,70 @@ DEV u32 net_of_port(const Params &P, u64 p, u32 dflt) {
   return net < P.n_nets ? net : dflt;
 }
 
+// Serving: a slot's arena is SERVE_SUB sub-arenas of `len` nodes, side by
+// side.  Sub-arena k has two words: words[2k] counts the nodes asked of it,
+// and never goes back while the slot's net runs; the one request that crosses
+// the end leaves what was left behind (first node << 32 | end) in words[2k+1],
+// where later requests that fit take from its front.  A request that does not
+// fit therefore changes nothing that another request counts on.  (Adding, and
+// giving back what did not fit, handed nodes out twice: with two such
+// requests under way, one's return brings the count back below the end while
+// it still holds the other's, and that one's return then takes away a third
+// request's nodes.)
+//
+// `n` consecutive nodes of a slot, from sub-arena k0 on; the first node's
+// place in the slot's arena, or NO_NODES.  One add where there is room; only
+// once sub-arena k0 is short are the others looked at, and nothing is refused
+// while a sub-arena changes hands.  No wave waits for another beyond the
+// store that leaves the rest.
+static const u64 NO_NODES = ~0ull;
+static const u32 SERVE_ROUNDS = 1u << 16;
+
+DEV u64 serve_add(u64 *words, u64 len, u32 k, u32 n) {
+  const u64 used = HVM_FAA(&words[2 * k], (u64)n);
+  if (used + n <= len) return k * len + used;
+  if (used <= len) HVM_ST(&words[2 * k + 1], used << 32 | len);
+  return NO_NODES;
+}
+
+DEV u64 serve_take(u64 *words, u64 len, u32 k0, u32 n) {
+  u64 at = NO_NODES;
+  if (n <= len) at = serve_add(words, len, k0 & (SERVE_SUB - 1), n);
+  bool moved = n <= len;
+  for (u32 round = 0; at == NO_NODES && moved && round < SERVE_ROUNDS; round++) {
+    moved = false;
+    for (u32 j = 0; j < SERVE_SUB && at == NO_NODES; j++) {
+      const u32 k = (k0 + j) & (SERVE_SUB - 1);
+      const u64 used = HVM_LD(&words[2 * k]);
+      if (used <= len) {
+        if (used + n <= len) {
+          at = serve_add(words, len, k, n);
+          moved = true;
+        }
+        continue;
+      }
+      u64 rest = HVM_LD(&words[2 * k + 1]);
+      const u64 pos = rest >> 32, end = rest & 0xFFFFFFFFull;
+      if (rest == 0) moved = true;  // on its way
+      else if (pos + n <= end) {
+        if (HVM_CAS(&words[2 * k + 1], &rest, rest + ((u64)n << 32))) at = k * len + pos;
+        moved = true;
+      }
+    }
+  }
+  return at;
+}
+
+// A slot's sub-arenas as they are before its net: nothing asked of any.
+DEV void serve_clear(u64 *words) {
+  for (u32 k = 0; k < 2 * SERVE_SUB; k++) HVM_ST(&words[k], 0ull);
+}
+
 // Serving: the lanes of a wave that take nodes together and are on the same
 // slot take them with one atomic add: exactly `need` nodes each, side by
 // side.  (Every serving lane takes at nearly every task, since its slot may
 // restart in between; with an atomic per lane the words of a few dozen slots
-// were the hottest lines of the launch.)  A slot's arena is SERVE_SUB
-// sub-arenas; the lane that adds goes through them in turn.
+// were the hottest lines of the launch.)
 // The lanes first find their slot's sum and their place in it, without a
 // memory access; then the first lane of every slot adds, all of them at once,
 // and the others take the result from it.  (Each slot's add waited for before
@@ -446,24 +504,13 @@ DEV void arena_room_serve(Lane &L, u32 need) {
     before = mine ? below : before;
     todo &= ~HVM_BALLOT(mine);
   }
-  u64 w = 0;
-  bool fits = false;
-  if (L.lane_id == lead) {
-    const u64 len = (u64)P.sub_granules << P.gran_shift;
-    u64 *const words = &P.arena_word[(u64)L.cur_net * SERVE_SUB];
-    // (a full sub-arena gives its add back and the next one is tried)
-    const u32 k0 = L.rw[RW_POPS] + lead;
-    for (u32 k = 0; k < SERVE_SUB && !fits; k++) {
-      u64 *const word = &words[(k0 + k) & (SERVE_SUB - 1)];
-      w = HVM_FAA(word, (u64)sum);
-      fits = (w & 0xFFFFFFFFull) + sum <= len;
-      if (!fits) HVM_FAA(word, (u64)0 - sum);
-    }
-    w = fits ? ((w >> 32) << P.gran_shift) + (w & 0xFFFFFFFFull) : ~0ull;
-  }
+  const u64 len = (u64)P.sub_granules << P.gran_shift;
+  u64 w = NO_NODES;
+  if (L.lane_id == lead) w = serve_take(&P.arena_word[(u64)L.cur_net * SERVE_WORDS], len, L.rw[RW_POPS] + lead, sum);
   w = lane_from(w, lead);
-  fits = w != ~0ull;
-  L.a_pos = fits ? w + before : 0;
+  const bool fits = w != NO_NODES;
+  const u64 slot0 = ((u64)P.serve_first << P.gran_shift) + (u64)L.cur_net * SERVE_SUB * len;
+  L.a_pos = fits ? slot0 + w + before : 0;
   L.a_end = fits ? L.a_pos + need : 0;
   if (!fits) fail(L, ERR_OOM, OOM_POOL);
 }
@@ -1408,8 +1455,7 @@ DEV void serve_complete(Lane &L, u32 s) {
   HVM_ST_SYS(e, idx + 1);
   // the slot again: its arena restarts (lanes drop their chunks at every
   // task, so no chunk of the old net is used again), then it is freed
-  for (u32 k = 0; k < SERVE_SUB; k++)
-    HVM_ST(&P.arena_word[s * SERVE_SUB + k], P.arena_base0[s * SERVE_SUB + k] << 32);
+  serve_clear(&P.arena_word[(u64)s * SERVE_WORDS]);
   publish();
   const u64 pos = HVM_FAA(&sv[SV_FREE_TAIL], 1ull);
   HVM_ST(&P.free_ring[pos % P.serve_slots], (u64)s + 1);

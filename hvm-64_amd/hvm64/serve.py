@@ -23,7 +23,7 @@ from . import Heap, HvmError, Host, Serving, arena_sizes, u24_port
 from . import configs
 
 NODE_BYTES = 16
-SUB_ARENAS = 8  # a slot's arena is cut in eight, taken from by lane index
+SUB_ARENAS = 8  # a slot's arena is cut in eight
 
 
 def slot_layout(heap_bytes, slot_nodes, slots):

@@ -230,8 +230,23 @@ struct Lane {
 // them when the wave's tasks have ended (lane_report).  Reporting on the
 // spot put a function call, and the register moves that a call's convention
 // asks for, behind every heap access.
+// (Bit 31: an address outside the heap was recorded before it.)
+static const u32 ERR_AFTER_BAD = 1u << 31;
 DEV void fail(Lane &L, u32 code, u32 site = 0) {
-  if (L.err == 0) L.err = code | site << 16;
+  if (L.err == 0) L.err = code | site << 16 | (L.bad ? ERR_AFTER_BAD : 0);
+}
+
+// Out of nodes.  Reported on the spot: the dump cell stands in for the missing
+// node, and what this lane and, once it has linked, others find there would
+// else be reported first, as an engine bug.  No call: the swap and the stores
+// stand at the ends of the allocation paths.
+DEV void out_of_nodes(Lane &L, u32 site = 0) {
+  u32 zero = 0;
+  if (HVM_CAS(&L.P->g->err, &zero, (u32)ERR_OOM)) {
+    HVM_ST(&L.P->g->err_info, site);
+    HVM_ST(&L.P->g->result, 0ull);
+  }
+  fail(L, ERR_OOM, site);
 }
 
 // The word at engine address `addr`; an address outside the heap is
@@ -250,8 +265,8 @@ DEV u64 xchg(Lane &L, u64 addr, u64 v) { return HVM_XCHG(hw(L, addr), v); }
 
 // Reports what the lane recorded (the first report of a launch is kept).
 DEV void lane_report(Lane &L) {
-  if (L.bad) report_error(L.P->g, ERR_BADPTR, BAD_HEAP_ADDR, L.bad);
-  if (L.err) report_error(L.P->g, L.err & 0xFFFF, L.err >> 16);
+  if (L.bad && (L.err == 0 || (L.err & ERR_AFTER_BAD))) report_error(L.P->g, ERR_BADPTR, BAD_HEAP_ADDR, L.bad);
+  else if (L.err) report_error(L.P->g, L.err & 0xFFFF, L.err >> 16);
   L.bad = 0;
   L.err = 0;
 }
@@ -327,7 +342,7 @@ DEV u64 alloc_lapped(Lane &L) {
       HVM_ST(heap + 2 * node, P_FREE);  // second word in use: not a free node
     }
   }
-  fail(L, ERR_OOM);
+  out_of_nodes(L);
   return dump_addr();
 }
 
@@ -524,7 +539,7 @@ DEV void arena_room_serve(Lane &L, u32 need) {
   const u64 slot0 = ((u64)P.serve_first << P.gran_shift) + (u64)L.cur_net * SERVE_SUB * len;
   L.a_pos = fits ? slot0 + w : 0;
   L.a_end = fits ? L.a_pos + need : 0;
-  if (!fits) fail(L, ERR_OOM, OOM_POOL);
+  if (!fits) out_of_nodes(L, OOM_POOL);
 }
 
 // Makes room for `need` consecutive nodes of the running task's net.  Right
@@ -550,7 +565,7 @@ DEV void arena_room(Lane &L, u32 need) {
   L.a_pos = c.pos;
   L.a_end = c.end;
   if (c.err) {
-    fail(L, c.err, c.site);
+    out_of_nodes(L, c.site);
     L.a_end = L.a_pos;  // every later allocation reports again
   }
 }

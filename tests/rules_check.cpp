@@ -80,10 +80,75 @@ static bool wide_definition() {
   return ok;
 }
 
+// The error reported is the one that came first.
+static bool first_error() {
+  bool ok = true;
+  for (u32 order = 0; order < 4; order++) {  // bit 0: a bad address first; bit 1: both kinds
+    Bench b;
+    const u64 bad = 0x20;
+    if (order & 1) hw(b.L, bad);
+    if (order != 1) fail(b.L, ERR_UNIMPL);
+    if (order == 2) hw(b.L, bad);
+    lane_report(b.L);
+    ok &= same("error", b.g.err, order & 1 ? ERR_BADPTR : ERR_UNIMPL);
+    ok &= same("address", b.g.result, order & 1 ? bad : 0);
+  }
+  return ok;
+}
+
+// A lane without a node reports it before anything can be found in the dump
+// cell: at once, in each way that nodes are allocated.
+static bool out_of_nodes_first() {
+  bool ok = true;
+  for (u32 way = 0; way < 3; way++) {
+    Bench b;
+    b.P.ov_nodes = 64;
+    b.P.ov_node0 = b.P.ring_node0 + b.P.wave_nodes - 64;
+    b.P.wave_nodes = 64;
+    u64 word = 1ull << 32, base0 = 1, pool_next = 2, ov_next = 256;
+    std::vector<u32> gmap(1 << 8, 0);
+    u32 len = 1;
+    u64 slot[SERVE_WORDS] = {};
+    if (way) {
+      b.P.gmap = gmap.data();
+      b.P.gmap_len = gmap.size();
+      b.P.gran_shift = 4;
+      b.P.n_nets = 1;
+      b.P.arena_word = way == 1 ? &word : slot;
+      b.P.arena_base0 = &base0;
+      b.P.arena_len = &len;
+      b.P.pool_next = &pool_next;
+      b.P.pool_end = 2;
+      b.P.ov_next = &ov_next;
+      b.P.ov_end = 256;
+      b.P.refill_granules = 1;
+      b.P.arena_chunk = 8;
+      b.P.sub_granules = 1;
+      b.P.serve_first = 1;
+    }
+    b.lane();
+    b.L.serve = way == 2;
+    u32 n = 0;
+    for (; n < 1000 && b.g.err == 0; n++) {
+      const u64 a = alloc_node(b.L);
+      if (a != dump_addr()) st2(b.L, a, P_NONE, P_NONE);
+    }
+    ok &= same("allocations until none is left", n < 1000, 1);
+    ok &= same("error", b.g.err, ERR_OOM);
+    ok &= same("site", b.g.err_info, way ? OOM_POOL : 0);
+    hw(b.L, 0x20);
+    lane_report(b.L);
+    ok &= same("error after a bad address", b.g.err, ERR_OOM);
+  }
+  return ok;
+}
+
 int main(int, char **argv) {
   const std::string c = argv[1];
   bool ok = false;
   if (c == "wide definition") ok = wide_definition();
+  if (c == "first error") ok = first_error();
+  if (c == "out of nodes first") ok = out_of_nodes_first();
   if (ok) std::printf("ok\n");
   return ok ? 0 : 1;
 }

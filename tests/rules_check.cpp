@@ -143,12 +143,37 @@ static bool out_of_nodes_first() {
   return ok;
 }
 
+// An access outside the heap is reported, whichever address it has: 0 too,
+// which the word of a freed cell holds.
+static bool outside_the_heap() {
+  bool ok = true;
+  Bench top;
+  const u64 end = HVM_HEAP_OFF + top.P.heap_words * 8;
+  for (u64 addr : {(u64)0, (u64)8, (u64)0x20, HVM_HEAP_OFF - 8, HVM_HEAP_OFF, end - 8, end, ADDR_MASK}) {
+    Bench b;
+    const bool out = addr < HVM_HEAP_OFF || addr >= end;
+    ok &= same("word", (u64)(hw(b.L, addr) - b.P.heap), out ? DUMP_WORD : (addr - HVM_HEAP_OFF) / 8);
+    lane_report(b.L);
+    ok &= same("error", b.g.err, out ? ERR_BADPTR : 0);
+    ok &= same("site", b.g.err_info, out ? BAD_HEAP_ADDR : 0);
+    ok &= same("address", b.g.result, out ? addr : 0);
+  }
+  Bench b;  // a wire whose cell was freed
+  const u64 cell = HVM_HEAP_OFF + RESERVED_WORDS * 8;
+  st(b.L, cell, P_FREE);
+  follow(b.L, wire_port(cell), true);
+  lane_report(b.L);
+  ok &= same("freed cell", b.g.err, ERR_BADPTR);
+  return ok;
+}
+
 int main(int, char **argv) {
   const std::string c = argv[1];
   bool ok = false;
   if (c == "wide definition") ok = wide_definition();
   if (c == "first error") ok = first_error();
   if (c == "out of nodes first") ok = out_of_nodes_first();
+  if (c == "outside the heap") ok = outside_the_heap();
   if (ok) std::printf("ok\n");
   return ok ? 0 : 1;
 }

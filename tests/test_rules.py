@@ -22,7 +22,7 @@ def rules(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["wide definition", "first error", "out of nodes first"])
+@pytest.mark.parametrize("case", ["wide definition", "first error", "out of nodes first", "outside the heap"])
 def test_rule(rules, case):
     r = subprocess.run([rules, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr

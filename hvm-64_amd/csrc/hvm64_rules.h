@@ -128,14 +128,15 @@ DEV u64 *hw(Lane &L, u64 addr);
 // gfx940 and later need two wait states before a VALU instruction may
 // overwrite the data registers of a store wider than 64 bits; the compiler
 // does not insert them after inline asm, so the asm ends with `s_nop 1`.
-// No memory clobber here and in the loads below: they are volatile, so they
-// keep their order among themselves and to publish(), and LDS accesses may
-// be scheduled around them.
+// The memory clobber, here and in the loads below, keeps them in order with
+// the relaxed atomics on the same words (a fresh var cell's store and a later
+// look at the cell); without it their order would rest on what the compiler
+// happens to do.
 DEV void st16(u64 *p, u64 w0, u64 w1) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef u64 u64x2 __attribute__((ext_vector_type(2)));
   const u64x2 d = {w0, w1};
-  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(d));
+  asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(d) : "memory");
 #else
   HVM_ST(p, w0);
   HVM_ST(p + 1, w1);
@@ -639,7 +640,8 @@ DEV void ld16x2(const u64 *p, const u64 *q, u64 &p0, u64 &p1, u64 &q0, u64 &q1) 
   u64x2 dp, dq;
   asm volatile("global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
                : "=&v"(dp), "=&v"(dq)
-               : "v"(p), "v"(q));
+               : "v"(p), "v"(q)
+               : "memory");
   p0 = dp.x;
   p1 = dp.y;
   q0 = dq.x;
@@ -655,7 +657,7 @@ DEV void ld16(const u64 *p, u64 &p0, u64 &p1) {
 #if defined(__HIP_DEVICE_COMPILE__)
   typedef u64 u64x2 __attribute__((ext_vector_type(2)));
   u64x2 dp;
-  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=v"(dp) : "v"(p));
+  asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=v"(dp) : "v"(p) : "memory");
   p0 = dp.x;
   p1 = dp.y;
 #else

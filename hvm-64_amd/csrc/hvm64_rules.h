@@ -222,9 +222,8 @@ struct Lane {
   // counters
   u32 rw[RW_SLOTS];
   // errors of this lane not yet reported (lane_report): the last address
-  // outside the heap, as its distance from the heap's start (0: none; address
-  // 0, which a freed word holds, counts), and the first other error's code
-  // and site
+  // outside the heap, bit 0 set (0: none; address 0, which a freed word holds,
+  // counts), and the first other error's code and site
   u64 bad;
   u32 err;
 };
@@ -259,7 +258,7 @@ DEV u64 *hw(Lane &L, u64 addr) {
   const Params &P = *L.P;
   const u64 off = addr - HVM_HEAP_OFF;
   const bool out = off >= P.heap_words * 8;
-  L.bad = out ? off : L.bad;
+  L.bad = out ? addr | 1 : L.bad;
   return (u64 *)((char *)P.heap + (out ? DUMP_WORD * 8 : off & ~7ull));
 }
 DEV u64 ld(Lane &L, u64 addr) { return HVM_LD(hw(L, addr)); }
@@ -269,7 +268,7 @@ DEV u64 xchg(Lane &L, u64 addr, u64 v) { return HVM_XCHG(hw(L, addr), v); }
 // Reports what the lane recorded (the first report of a launch is kept).
 DEV void lane_report(Lane &L) {
   if (L.bad && (L.err == 0 || (L.err & ERR_AFTER_BAD)))
-    report_error(L.P->g, ERR_BADPTR, BAD_HEAP_ADDR, L.bad + HVM_HEAP_OFF);
+    report_error(L.P->g, ERR_BADPTR, BAD_HEAP_ADDR, L.bad & ~1ull);
   else if (L.err) report_error(L.P->g, L.err & 0xFFFF, L.err >> 16);
   L.bad = 0;
   L.err = 0;

@@ -573,18 +573,29 @@ DEV void arena_room(Lane &L, u32 need) {
   }
 }
 
-// `need` (at most N) nodes: out[0 .. need).  From the free cache, newest
-// first, then from the slice's first lap; both are address arithmetic
-// without a branch.  Past the first lap one by one, in a loop, so that the
-// scan is in the code once per call site.
+// `need` (at most N) nodes, each on its own: out[0 .. need).  From the free
+// cache, newest first, then from the slice's first lap; both are address
+// arithmetic without a branch.  Past the first lap one by one, in a loop, so
+// that the scan is in the code once per call site.
 template <u32 N>
 DEV void alloc_nodes(Lane &L, u32 need, u64 (&out)[N]) {
   if (L.arenas) {
-    if (need) arena_room(L, need);
-    const bool ok = L.a_pos + need <= L.a_end;
+    // the last nodes of a chunk that holds fewer than `need`, then the next
+    // chunk's (a serving lane has no chunk: it takes what it needs)
+    u32 rest = 0;
+    const u64 last = L.a_pos;
+    if (!L.serve) {
+      const u64 left = L.a_net == L.cur_net ? L.a_end - L.a_pos : 0;
+      rest = left < need ? (u32)left : 0;
+      L.a_pos += rest;
+    }
+    const u32 more = need - rest;
+    if (more) arena_room(L, more);
+    const bool ok = L.a_pos + more <= L.a_end;
 #pragma unroll
-    for (u32 j = 0; j < N; j++) out[j] = ok ? HVM_HEAP_OFF + (L.a_pos + j) * 16 : dump_addr();
-    L.a_pos += ok ? need : 0;
+    for (u32 j = 0; j < N; j++)
+      out[j] = j < rest || ok ? HVM_HEAP_OFF + ((j < rest ? last : L.a_pos - rest) + j) * 16 : dump_addr();
+    L.a_pos += ok ? more : 0;
     return;
   }
   const u32 used = L.in_lds ? (L.fcn < need ? L.fcn : need) : 0;

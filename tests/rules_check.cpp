@@ -167,6 +167,41 @@ static bool outside_the_heap() {
   return ok;
 }
 
+// A lane of a planned batch hands out every node of its chunks, in order,
+// whatever the sizes of its requests: the chunks (8 nodes after the first few)
+// end within requests of 1 to 6 nodes.
+static bool arena_remainders() {
+  bool ok = true;
+  for (u32 first = 1; first <= 6; first++) {
+    Bench b;
+    const u64 nodes = 214;
+    u64 word = 1ull << 32, base0 = 1, pool_next = 1 + nodes / 2, ov_next = 1000;
+    std::vector<u32> gmap(1 << 10, 0);
+    u32 len = nodes / 2;
+    b.P.gmap = gmap.data();
+    b.P.gmap_len = gmap.size();
+    b.P.gran_shift = 1;
+    b.P.n_nets = 1;
+    b.P.arena_word = &word;
+    b.P.arena_base0 = &base0;
+    b.P.arena_len = &len;
+    b.P.pool_next = &pool_next;
+    b.P.pool_end = pool_next;
+    b.P.ov_next = &ov_next;
+    b.P.ov_end = 1000;
+    b.P.refill_granules = 4;
+    b.P.arena_chunk = 8;
+    b.lane();
+    for (u64 at = 0, need = first; at + need + 8 <= nodes; at += need, need = need % 6 + 1) {
+      u64 out[6];
+      alloc_nodes(b.L, (u32)need, out);
+      for (u64 j = 0; j < need; j++) ok &= same("node", out[j], HVM_HEAP_OFF + (2 + at + j) * 16);
+    }
+    ok &= same("error", b.g.err, 0);
+  }
+  return ok;
+}
+
 int main(int, char **argv) {
   const std::string c = argv[1];
   bool ok = false;
@@ -174,6 +209,7 @@ int main(int, char **argv) {
   if (c == "first error") ok = first_error();
   if (c == "out of nodes first") ok = out_of_nodes_first();
   if (c == "outside the heap") ok = outside_the_heap();
+  if (c == "arena remainders") ok = arena_remainders();
   if (ok) std::printf("ok\n");
   return ok ? 0 : 1;
 }

@@ -22,7 +22,8 @@ def rules(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["wide definition", "first error", "out of nodes first", "outside the heap"])
+@pytest.mark.parametrize("case", ["wide definition", "first error", "out of nodes first", "outside the heap",
+                                  "arena remainders"])
 def test_rule(rules, case):
     r = subprocess.run([rules, case], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout == "ok\n", r.stdout + r.stderr

@@ -1350,10 +1350,11 @@ int hvm_gpu_normal(hvm_gpu *h) {
     Params P = make_params(h, ~0ull);
     // (an error of the expansion ends the reduction at its first look)
     hip_check(launch_expand(P, h->root_cell, h->stream), "launch expand");
+    h->last.root = 0;  // until the control block has come back
     try {
       run_reduce(h, ~0ull, false, true);
     } catch (Error &) {
-      h->root_cell = h->last.root;
+      if (h->last.root) h->root_cell = h->last.root;
       throw;
     }
     h->root_cell = h->last.root;

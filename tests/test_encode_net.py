@@ -4,17 +4,12 @@ definitions.  On the CPU through the engine's own host code and a one-lane
 device (tests/fake_device.cpp), which sees a register written outside its
 area; on the GPU through the package.  Rewrite counts (and on the GPU normal
 forms) are the oracle's, and the same handle boots a definition afterwards."""
-import os
 import random
-import shutil
 import subprocess
 
 import pytest
 
-HERE = os.path.dirname(os.path.abspath(__file__))
-ROOT = os.path.dirname(HERE)
-CSRC = os.path.join(ROOT, "hvm-64_amd", "csrc")
-HIP = "/opt/rocm/include"
+import fake_device
 
 BOOK = """@add = ($([+] $(a b)) (a b))
 @mul = ($([*] $(a b)) (a b))
@@ -48,17 +43,7 @@ NETS.update({f"nest {n}": nest(n) for n in (9, 10, 11, 14, 16, 17, 30)})
 
 @pytest.fixture(scope="module")
 def encode_check(tmp_path_factory):
-    gxx = shutil.which("g++")
-    if gxx is None or not os.path.exists(os.path.join(HIP, "hip", "hip_runtime.h")):
-        pytest.skip("g++ or the HIP headers not available")
-    out = tmp_path_factory.mktemp("encode")
-    flags = ["-O1", "-w", "-std=c++17", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I", HIP, "-I", CSRC, "-I",
-             os.path.join(ROOT, "include"), "-I", HERE]
-    src = [os.path.join(CSRC, f"hvm64_{x}.cpp") for x in ("api", "host", "defcomp")]
-    src += [os.path.join(HERE, f) for f in ("fake_device.cpp", "encode_check.cpp")]
-    exe = str(out / "encode_check")
-    subprocess.run([gxx] + flags + src + ["-o", exe], check=True)
-    return exe
+    return fake_device.build("encode_check", tmp_path_factory.mktemp("encode"))
 
 
 @pytest.mark.parametrize("compiled", [1, 0])

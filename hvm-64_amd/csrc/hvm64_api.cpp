@@ -204,11 +204,13 @@ Params make_params(hvm_gpu *h, u64 limit) {
 // Waits for the stream and takes over the control block, which the last
 // kernel has copied to the host (mirrored) or a kernel of its own does.
 void sync_globals(hvm_gpu *h, bool mirrored = false) {
+  const bool unknown = h->ring_unknown;
+  h->ring_unknown = true;  // should the block not come back
   if (!mirrored) hip_check(launch_mirror(make_params(h, ~0ull), h->stream), "launch mirror");
   hip_check(hipStreamSynchronize(h->stream), "kernel");
   std::memcpy(&h->last, h->pin, sizeof(Globals));
+  h->ring_unknown = unknown || h->last.err != 0;
   if (h->last.err) {
-    h->ring_unknown = true;
     u32 e = h->last.err;
     int code = e == ERR_OOM ? HVM_E_OOM
                : e == ERR_UNIMPL ? HVM_E_UNIMPL_PAIR

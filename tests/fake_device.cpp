@@ -21,6 +21,7 @@ const u32 GUARD_WORDS = 64 * 64;
 std::vector<u64> chip_regs(LDS_SLOTS * 64 + GUARD_WORDS, GUARD);
 pair chip_links[LINK_CAP * 64];
 int sync_failures = 0;
+Params ring;  // the ring of the last launch that used it
 
 // A lane as a one-wave kernel sets it up: `regs`: with registers on chip.
 void lane_on_chip(Lane &L, const Params &P, bool regs) {
@@ -41,6 +42,11 @@ bool fake_guard_intact() {
   return true;
 }
 void fake_fail_next_sync() { sync_failures = 1; }
+bool fake_ring_clear() {
+  for (u64 i = 0; i < 1024; i++)  // (a test's redexes are in its first slots)
+    if (ring.queue[2 * i] || ring.queue[2 * i + 1]) return false;
+  return true;
+}
 
 // ---------------------------------------------------------------------------
 // launches
@@ -90,6 +96,7 @@ hipError_t launch_reset(const Params &P, u64 q0, u64 q1, hipStream_t) {
   return hipSuccess;
 }
 hipError_t launch_reduce(const Params &P, u32, hipStream_t) {
+  ring = P;
   Lane L;
   lane_on_chip(L, P, true);
   while (P.g->q_head < P.g->q_tail && P.g->err == 0 && P.g->done < P.limit) {

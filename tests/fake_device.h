@@ -5,3 +5,5 @@
 bool fake_guard_intact();
 // The next wait for the stream fails.
 void fake_fail_next_sync();
+// The global redex ring holds no redex.
+bool fake_ring_clear();

@@ -1,4 +1,4 @@
-"""A handle's root cell after a Net::normal whose launch the host lost
+"""A handle after launches the host lost: its root cell and its redex ring
 (tests/handle_check.cpp).  CPU only: the engine's host code on a one-lane
 device in host memory."""
 import subprocess

@@ -83,7 +83,7 @@ enum : u32 {
 enum : u32 { OOM_POOL = 1, OOM_OVERFLOW = 2 };
 
 // Which consistency check reported ERR_BADPTR (Globals::err_info).
-enum : u32 { BAD_HEAP_ADDR = 1, BAD_LINK_LIST, BAD_CHAIN, BAD_RESOLVE, BAD_SLOTS, BAD_DEF_CALL, BAD_DEF_EXPAND,
+enum : u32 { BAD_HEAP_ADDR = 1, BAD_CHAIN = 3, BAD_RESOLVE, BAD_SLOTS, BAD_DEF_CALL, BAD_DEF_EXPAND,
              BAD_NET };  // BAD_NET: a port beyond the granule map
 
 // Scheduler statistics (summed over waves): iterations with work, idle

@@ -676,13 +676,6 @@ DEV void ld16(const u64 *p, u64 &p0, u64 &p1) {
 #endif
 }
 
-// A fresh pair of var cells (both words of one node): cells n and n + 8.
-DEV u64 alloc_vars2(Lane &L) {
-  u64 n = alloc_node(L);
-  st2(L, n, P_NONE, P_NONE);
-  return n;
-}
-
 // One fresh var cell; the node's other word stays FREE.
 DEV u64 alloc_var1(Lane &L) {
   u64 n = alloc_node(L);
@@ -1542,8 +1535,6 @@ DEV void serve_settle(Lane &L) {
   if (L.acct_delta != 0 && L.acct_old + L.acct_delta == 0) serve_complete(L, L.acct_net);
   L.acct_delta = 0;
 }
-
-static const u32 NO_DEF = 0xFFFFFFFFu;
 
 DEV Interp interp_none(const Lane &L) {
   Interp I;

@@ -112,9 +112,9 @@ class Server:
         book, self.table = configs.mix_book(variants, book_seed)
         self.host = Host(book, self.heap)
         if slot_nodes is None:
-            # every variant alone, allocation counted; lanes take nodes in
-            # chunks (a serving lane drops its chunk at every task), so a
-            # slot holds twice the largest count (1.3 times ran dry)
+            # every variant alone, allocation counted; a slot holds twice the
+            # largest count.  (Takes are exact: with 1.02 times the count 128
+            # requests on 24 slots take the same 125 ms.)
             defs = [self.host.defs[self.table[v][0]] for v in variants]
             slot_nodes = 2 * max(arena_sizes(self.heap, defs, margin=1.0, extra=0)) + 4096
         self.slot_nodes = slot_nodes
